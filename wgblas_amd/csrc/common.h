@@ -18,8 +18,8 @@ struct wgb_ctx {
   bool timed_once = false;
   float last_ms = 0.0f;
   int num_cus = 0;
-  // Device scratch for the two-pass reductions: per-block partials followed
-  // by a result slot. Stream order makes reuse across calls safe.
+  // Device scratch for the reductions: per-block partials followed by the
+  // arrival counter. Stream order makes reuse across calls safe.
   void *scratch = nullptr;
   size_t scratch_bytes = 0;
   // GEMM split-k workspace: partial tiles of the launch's last, partly
@@ -30,8 +30,10 @@ struct wgb_ctx {
   // its copy of B (grown on demand, reused in stream order).
   void *op_ws = nullptr;
   size_t op_ws_bytes = 0;
-  // Pinned host slot the host-result reductions copy their scalar into.
+  // Pinned host slot the host-result reductions store their scalar into, and
+  // the number of the last such call.
   void *host_result = nullptr;
+  uint32_t host_seq = 0;
   char name[256] = {0};
   char arch[64] = {0};
 };
@@ -53,9 +55,9 @@ void timing_begin(wgb_ctx *ctx);
 void timing_end(wgb_ctx *ctx);
 
 // Largest number of first-pass blocks a reduction may use; the scratch
-// buffer is sized for this many 32-byte partials plus the result slot.
+// buffer is sized for this many 32-byte partials plus the arrival counter.
 constexpr int kMaxReduceBlocks = 4096;
-constexpr size_t kScratchBytes = (size_t)kMaxReduceBlocks * 32 + 256;  // 32-byte partial slots + result
+constexpr size_t kScratchBytes = (size_t)kMaxReduceBlocks * 32 + 256;  // 32-byte partial slots + counter
 
 // Grows the context's operand workspace (ctx->op_ws) to at least `bytes`;
 // the stream is drained first, since an earlier launch may still read it.

@@ -17,8 +17,11 @@
 //    strides read one element per lane;
 //  * a block folds its lanes with 64-lane shuffles, then its four waves in
 //    LDS, in a fixed order, and stores one partial;
-//  * stage 2 (one block, a second launch) folds the G partials in a fixed
-//    order and applies the final combine (snrm2) or index pick (isamax).
+//  * stage 2 folds the G partials in a fixed order and applies the final
+//    combine (snrm2) or index pick (isamax): in the last block of the same
+//    launch for few blocks, else in one block of a second launch;
+//  * a host result is stored by the folding block to pinned host memory, with
+//    the call's number behind it, which the host reads.
 //
 // The per-element arithmetic follows the WGSL kernels: f32 accumulation,
 // snrm2's big/medium/small classification with the same power-of-two
@@ -32,6 +35,7 @@
 // (wgblas moves them to fit double-double's f32 exponent range).
 #include "common.h"
 
+#include <chrono>
 #include <type_traits>
 
 namespace {
@@ -60,7 +64,14 @@ constexpr int kThreads = 256;
 // blocks, +1-2.5% (sdot 6.97, sasum 6.86, snrm2 6.86, isamax 6.81 TB/s;
 // the box's read roof measured by roof_probe: 7.1 TB/s).
 constexpr int kUnroll = 16;
+constexpr int kTail = 4;  // loads in flight over what is left of a range
 constexpr int64_t kElemsPerBlockMin = 4096;
+// Up to this many first-pass blocks the last one to arrive folds (one launch).
+// The arrivals serialise on one word, about 10 ns each, against about 2 us
+// for the second launch: four reductions of fp32 vectors, both ways, 245 blocks
+// (n = 10^6) 26.3 us fused and 29.9 in two launches, 977 blocks (4 10^6) 62.8
+// and 29.1, 4096 blocks (2^28) 911 and 770.
+constexpr int kMaxFusedBlocks = 256;
 
 // snrm2 thresholds and scales (powers of two): src/shaders/snrm2.wgsl:33-36.
 constexpr float kTsml = 0x1p-63f;
@@ -76,6 +87,12 @@ constexpr double kDTsml = 0x1p-511;
 constexpr double kDTbig = 0x1p486;
 constexpr double kDSsml = 0x1p537;
 constexpr double kDSbig = 0x1p-538;
+
+// Host-result calls: the pinned slot's word that holds the number of the call
+// whose result is there, and how long the host reads it before it waits for the
+// stream.
+constexpr int kSeqWord = 8;
+constexpr int kSpinMicros = 100;
 
 // Partial slots in the context scratch (the largest Partial is dnrm2's).
 constexpr size_t kPartialBytes = 32;
@@ -431,13 +448,92 @@ __device__ __forceinline__ void chunk_of(int64_t total, int64_t &beg, int64_t &e
   if (beg > end) beg = end;
 }
 
-// A block's partial goes to its slot; stage 2 (fold_kernel) folds them.
-// (Folding in the last block of the same launch needs an agent-scope
-// release per block, which writes back the XCD's L2: measured ~90 us per
-// 2048-block launch on MI355X, far more than the second launch costs.)
+// Where a result goes. seq != 0: ptr is the context's pinned host slot, and the
+// host waits for seq in the word behind it.
 template <class Op>
-__device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Partial *partials) {
-  if (threadIdx.x == 0) partials[blockIdx.x] = p;
+struct Output {
+  typename Op::Result *ptr;
+  uint32_t seq;
+};
+
+// The result, then (system-scope words, in order: the first has left before the
+// second is issued) the sequence number.
+template <class Op>
+__device__ __forceinline__ void store_result(const typename Op::Partial &p, Output<Op> out) {
+  const typename Op::Result r = Op::result(p);
+  if (out.seq == 0) {
+    *out.ptr = r;
+    return;
+  }
+  uint32_t w[sizeof(r) / 4];
+  __builtin_memcpy(w, &r, sizeof(r));
+#pragma unroll
+  for (size_t i = 0; i < sizeof(r) / 4; ++i)
+    __hip_atomic_store(reinterpret_cast<uint32_t *>(out.ptr) + i, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __hip_atomic_store(reinterpret_cast<uint32_t *>(out.ptr) + kSeqWord, out.seq, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Partials cross XCDs (each with its own L2) inside one launch as relaxed
+// agent-scope atomic words: such stores and loads go past the L2s, so no
+// cache has to be written back or invalidated.
+template <typename P>
+__device__ __forceinline__ void store_partial(P *slot, const P &p) {
+  static_assert(sizeof(P) % 4 == 0, "partials are whole words");
+  uint32_t w[sizeof(P) / 4];
+  __builtin_memcpy(w, &p, sizeof(P));
+#pragma unroll
+  for (size_t i = 0; i < sizeof(P) / 4; ++i)
+    __hip_atomic_store(reinterpret_cast<uint32_t *>(slot) + i, w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename P>
+__device__ __forceinline__ P load_partial(const P *slot) {
+  uint32_t w[sizeof(P) / 4];
+#pragma unroll
+  for (size_t i = 0; i < sizeof(P) / 4; ++i)
+    w[i] = __hip_atomic_load(reinterpret_cast<const uint32_t *>(slot) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  P p;
+  __builtin_memcpy(&p, w, sizeof(P));
+  return p;
+}
+
+// A block's partial goes to its slot. With at most kMaxFusedBlocks blocks
+// (`out` given) the block that arrives last folds them all in the same
+// launch, in fold_kernel's order; otherwise stage 2 (fold_kernel) does.
+// The arrival is ordered after the partial by waiting for the stores
+// (s_waitcnt vmcnt(0)): a release fence at agent scope would write back the
+// XCD's L2 in every block (~90 us per 2048-block launch on MI355X).
+// The last block sets the counter back to 0 for the stream's next launch.
+template <class Op>
+__device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Partial *partials,
+                                       uint32_t *arrived, Output<Op> out) {
+  if (!out.ptr) {
+    if (threadIdx.x == 0) partials[blockIdx.x] = p;
+    return;
+  }
+  __shared__ bool last;
+  if (threadIdx.x == 0) {
+    last = gridDim.x == 1;
+    if (!last) {
+      store_partial(partials + blockIdx.x, p);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      last = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+  }
+  __syncthreads();
+  if (!last) return;
+  if (gridDim.x > 1) {
+    p = threadIdx.x < gridDim.x ? load_partial(partials + threadIdx.x) : Op::identity();
+    for (uint32_t i = threadIdx.x + kThreads; i < gridDim.x; i += kThreads)
+      p = Op::merge(p, load_partial(partials + i));
+    p = block_merge<Op>(p);
+  }
+  if (threadIdx.x == 0) {
+    if (gridDim.x > 1) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    store_result<Op>(p, out);
+  }
 }
 
 // Unit-stride, 16-byte-aligned operands: 16-byte non-temporal loads,
@@ -445,7 +541,8 @@ __device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Part
 template <class Op>
 __global__ __launch_bounds__(kThreads) void reduce_vec(const typename Op::Elem *__restrict__ x,
                                                        const typename Op::Elem *__restrict__ y, int64_t n,
-                                                       typename Op::Partial *__restrict__ partials) {
+                                                       typename Op::Partial *__restrict__ partials,
+                                                       uint32_t *arrived, Output<Op> out) {
   typedef typename Op::V V;
   constexpr int W = Vec16<typename Op::Elem>::W;
   const V *xv = reinterpret_cast<const V *>(x);
@@ -465,6 +562,17 @@ __global__ __launch_bounds__(kThreads) void reduce_vec(const typename Op::Elem *
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) Op::addv(s, a[u], b[u], W * (q + u * kThreads));
   }
+  // what is left (a short vector's whole share), kTail loads in flight
+  for (; q + (kTail - 1) * kThreads < end; q += kTail * kThreads) {
+    V a[kTail], b[kTail];
+#pragma unroll
+    for (int u = 0; u < kTail; ++u) {
+      a[u] = xv[q + u * kThreads];
+      b[u] = Op::NIN == 2 ? yv[q + u * kThreads] : a[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kTail; ++u) Op::addv(s, a[u], b[u], W * (q + u * kThreads));
+  }
   for (; q < end; q += kThreads) {
     V a = xv[q];
     Op::addv(s, a, Op::NIN == 2 ? yv[q] : a, W * q);
@@ -473,7 +581,7 @@ __global__ __launch_bounds__(kThreads) void reduce_vec(const typename Op::Elem *
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
     for (int64_t i = nv * W; i < n; ++i)
       Op::add1(s, x[i], Op::NIN == 2 ? y[i] : (typename Op::Elem)0, i, 0);
-  finish<Op>(block_merge<Op>(Op::finish(s)), partials);
+  finish<Op>(block_merge<Op>(Op::finish(s)), partials, arrived, out);
 }
 
 // Whether Op has add_kept (a vector of which some elements are kept).
@@ -507,7 +615,8 @@ __device__ __forceinline__ uint32_t kept_mask(uint32_t v) {
 template <class Op, int INC>
 __global__ __launch_bounds__(kThreads) void reduce_span(const typename Op::Elem *__restrict__ x,
                                                         const typename Op::Elem *__restrict__ y, int64_t n,
-                                                        typename Op::Partial *__restrict__ partials) {
+                                                        typename Op::Partial *__restrict__ partials,
+                                                       uint32_t *arrived, Output<Op> out) {
   typedef typename Op::V V;
   constexpr int W = Vec16<typename Op::Elem>::W;
   const V *xv = reinterpret_cast<const V *>(x);
@@ -552,7 +661,7 @@ __global__ __launch_bounds__(kThreads) void reduce_span(const typename Op::Elem 
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
     for (uint32_t e = (uint32_t)nv * W; e < span; ++e)
       if (e % INC == 0) Op::add1(s, x[e], Op::NIN == 2 ? y[e] : (typename Op::Elem)0, e / INC, 0);
-  finish<Op>(block_merge<Op>(Op::finish(s)), partials);
+  finish<Op>(block_merge<Op>(Op::finish(s)), partials, arrived, out);
 }
 
 // Any positive strides (and misaligned unit stride): one element per lane
@@ -562,7 +671,8 @@ __global__ __launch_bounds__(kThreads) void reduce_strided(const typename Op::El
                                                            int64_t incx,
                                                            const typename Op::Elem *__restrict__ y,
                                                            int64_t incy, int64_t n,
-                                                           typename Op::Partial *__restrict__ partials) {
+                                                           typename Op::Partial *__restrict__ partials,
+                                                           uint32_t *arrived, Output<Op> out) {
   typedef typename Op::Elem T;
   int64_t beg, end;
   chunk_of(n, beg, end);
@@ -579,14 +689,14 @@ __global__ __launch_bounds__(kThreads) void reduce_strided(const typename Op::El
     for (int u = 0; u < kUnroll; ++u) Op::add1(s, a[u], b[u], i + u * kThreads, u & 3);
   }
   for (; i < end; i += kThreads) Op::add1(s, x[i * incx], Op::NIN == 2 ? y[i * incy] : (T)0, i, 0);
-  finish<Op>(block_merge<Op>(Op::finish(s)), partials);
+  finish<Op>(block_merge<Op>(Op::finish(s)), partials, arrived, out);
 }
 
 // Stage 2: one block folds the G partials in a fixed order (each thread
 // issues all of its loads before folding them) and writes the result.
 template <class Op>
 __global__ __launch_bounds__(kThreads) void fold_kernel(const typename Op::Partial *__restrict__ partials,
-                                                        int G, typename Op::Result *__restrict__ out) {
+                                                        int G, Output<Op> out) {
   constexpr int kPer = wgb::kMaxReduceBlocks / kThreads;
   typename Op::Partial v[kPer];
 #pragma unroll
@@ -598,7 +708,7 @@ __global__ __launch_bounds__(kThreads) void fold_kernel(const typename Op::Parti
 #pragma unroll
   for (int r = 1; r < kPer; ++r) p = Op::merge(p, v[r]);
   p = block_merge<Op>(p);
-  if (threadIdx.x == 0) *out = Op::result(p);
+  if (threadIdx.x == 0) store_result<Op>(p, out);
 }
 
 // v * 2^e by editing the exponent field, as scaledSum.wgsl's ldexpBits does:
@@ -691,14 +801,16 @@ int check_vec(int64_t n, const T *x, int64_t incx, const char *xname, const char
 }
 
 void *partials_of(wgb_ctx *ctx) { return ctx->scratch; }
-void *result_slot(wgb_ctx *ctx) {
+// Behind the partials; wgb_init clears it.
+void *arrival_counter(wgb_ctx *ctx) {
   return (char *)ctx->scratch + (size_t)wgb::kMaxReduceBlocks * kPartialBytes;
 }
 
-// Stage 1 (the read pass) and stage 2 (the fold), two launches on the stream.
+// Stage 1 (the read pass) and stage 2 (the fold): one launch for few blocks,
+// else two on the stream.
 template <class Op>
 int launch_reduce(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t incx,
-                  const typename Op::Elem *y, int64_t incy, typename Op::Result *d_out,
+                  const typename Op::Elem *y, int64_t incy, Output<Op> out,
                   const char *what) {
   static_assert(sizeof(typename Op::Partial) <= kPartialBytes, "partial slot too small");
   const int G = reduce_blocks(n);
@@ -706,33 +818,28 @@ int launch_reduce(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t i
   int Gl = G;
   const bool same = Op::NIN == 1 || (incy == incx && aligned16(y));
   const int64_t span = (n - 1) * incx + 1;
+  auto *arrived = (uint32_t *)arrival_counter(ctx);
+  const Output<Op> unfused = {nullptr, 0};
+  Output<Op> fused = G <= kMaxFusedBlocks ? out : unfused;
   if (incx == 1 && aligned16(x) && same) {
-    reduce_vec<Op><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part);
+    reduce_vec<Op><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
   } else if (incx >= 2 && incx <= 4 && aligned16(x) && same && span < ((int64_t)1 << 31)) {
     // G from the span, not n: each block reads a span range.
     Gl = reduce_blocks(span);
+    fused = Gl <= kMaxFusedBlocks ? out : unfused;
     if (incx == 2)
-      reduce_span<Op, 2><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part);
+      reduce_span<Op, 2><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
     else if (incx == 3)
-      reduce_span<Op, 3><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part);
+      reduce_span<Op, 3><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
     else
-      reduce_span<Op, 4><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part);
+      reduce_span<Op, 4><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
   } else {
-    reduce_strided<Op><<<G, kThreads, 0, ctx->stream>>>(x, incx, y, incy, n, part);
+    reduce_strided<Op><<<G, kThreads, 0, ctx->stream>>>(x, incx, y, incy, n, part, arrived, fused);
   }
   WGB_CHECK_LAUNCH(what);
-  fold_kernel<Op><<<1, kThreads, 0, ctx->stream>>>(part, Gl, d_out);
+  if (fused.ptr) return WGB_OK;
+  fold_kernel<Op><<<1, kThreads, 0, ctx->stream>>>(part, Gl, out);
   WGB_CHECK_LAUNCH(what);
-  return WGB_OK;
-}
-
-// Copies a device scalar into the context's pinned slot and waits for it.
-template <typename T>
-int fetch_scalar(wgb_ctx *ctx, const T *d_src, T *host_dst) {
-  WGB_CHECK_HIP(hipMemcpyAsync(ctx->host_result, d_src, sizeof(T), hipMemcpyDeviceToHost,
-                               ctx->stream));
-  WGB_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  *host_dst = *(const T *)ctx->host_result;
   return WGB_OK;
 }
 
@@ -755,9 +862,28 @@ int reduce_to_device(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_
   wgb::timing_begin(ctx);
   if (n <= 0)
     set_value<<<1, 1, 0, ctx->stream>>>(d_result, empty);
-  else if ((st = launch_reduce<Op>(ctx, n, x, incx, y, incy, d_result, what)))
+  else if ((st = launch_reduce<Op>(ctx, n, x, incx, y, incy, Output<Op>{d_result, 0}, what)))
     return st;
   wgb::timing_end(ctx);
+  return WGB_OK;
+}
+
+// Waits for call `seq`'s number in the host slot (four reductions of 100 003
+// floats, host results: copy command and stream wait 76.2 us, stream wait alone
+// 65.4, this 45.9): read directly for as long as a
+// short reduction takes, then (and after an error on the stream, when it never
+// comes) by waiting for the stream, whose own wait costs several us more.
+template <class Op>
+int await_result(wgb_ctx *ctx, uint32_t seq, typename Op::Result *result) {
+  typedef std::chrono::steady_clock Clock;
+  const uint32_t *word = (const uint32_t *)ctx->host_result + kSeqWord;
+  const auto until = Clock::now() + std::chrono::microseconds(kSpinMicros);
+  bool there = false;
+  do {
+    for (int i = 0; i < 64 && !there; ++i) there = __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq;
+  } while (!there && Clock::now() < until);
+  if (!there) WGB_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  *result = *(const typename Op::Result *)ctx->host_result;
   return WGB_OK;
 }
 
@@ -779,11 +905,15 @@ int reduce_to_host(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t 
     y = x;
     incy = incx;
   }
-  auto *slot = (typename Op::Result *)result_slot(ctx);
+  // The last block stores the result and this call's number to the context's
+  // pinned (coherent) host slot itself: no copy command behind the kernels.
+  auto *slot = (typename Op::Result *)ctx->host_result;
+  if (++ctx->host_seq == 0) ctx->host_seq = 1;
+  const uint32_t seq = ctx->host_seq;
   wgb::timing_begin(ctx);
-  if ((st = launch_reduce<Op>(ctx, n, x, incx, y, incy, slot, what))) return st;
+  if ((st = launch_reduce<Op>(ctx, n, x, incx, y, incy, Output<Op>{slot, seq}, what))) return st;
   wgb::timing_end(ctx);
-  return fetch_scalar(ctx, slot, result);
+  return await_result<Op>(ctx, seq, result);
 }
 
 }  // namespace

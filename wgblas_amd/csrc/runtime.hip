@@ -119,7 +119,11 @@ extern "C" int wgb_init(int device, wgb_ctx **out) {
   if (e == hipSuccess) e = hipEventCreate(&ctx->ev_stop);
   if (e == hipSuccess) e = hipMalloc(&ctx->scratch, wgb::kScratchBytes);
   if (e == hipSuccess) ctx->scratch_bytes = wgb::kScratchBytes;
+  // the reductions' arrival counter starts at 0
+  if (e == hipSuccess) e = hipMemsetAsync(ctx->scratch, 0, wgb::kScratchBytes, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e == hipSuccess) e = hipHostMalloc(&ctx->host_result, 64, hipHostMallocDefault);
+  if (e == hipSuccess) std::memset(ctx->host_result, 0, 64);
   if (e != hipSuccess) {
     int st = wgb::fail_hip(e, "wgb_init");
     wgb_destroy(ctx);
