@@ -8,10 +8,10 @@
 //
 // Both forms read A once and are HBM-bound. A lane's loads are 4 consecutive
 // elements (16 bytes in fp32, 32 in fp64).
-//   N: a lane owns 4 consecutive rows in each of kGroupsN 1024-row groups
-//      (one 4-element load per group and column, kStepN columns per step), and a
-//      block walks a long run of columns (few, deep blocks); the
-//      columns are walked in order and a column whose x entry is zero is
+//   N: a lane owns 4 consecutive rows (one 4-element load per column, kStepN
+//      columns per step), and a block walks a long run of columns (few, deep
+//      blocks; where those are too few, narrower ones whose waves share the
+//      columns); a column whose x entry is zero is
 //      skipped, as reference BLAS does for this form (so 0 * Inf or 0 * NaN
 //      in that column never reaches y).
 //   T: a wave owns 8 columns (4 for short columns) and walks the rows 512
@@ -49,9 +49,16 @@ constexpr int64_t kShortColsRows = 4096;
 // with 2048 blocks of 64 columns (16384^2: 6.24 against 5.77 TB/s); fewer
 // splits also mean fewer partial sums to write and fold.
 constexpr int kStepN = 8;
-constexpr int kGroupsN = 1;
 constexpr int kTargetBlocksN = 256;
 constexpr int kMinColsN = 256;
+// Where those blocks would be fewer than the target (below 8192 x 8192):
+// blocks of 256 rows whose kColWaves waves share at least kMinColsNarrow
+// columns, partial sums added in LDS. 4096^2, fp32: 64 wide blocks 38.2 us, 256
+// narrow ones 12.9 (5.2 TB/s; 4 waves 16.4); fp64 70.2 and 27.1. Splits of at
+// least 64 / 128 / 256 columns: fp32 512^2 6.9 / 6.6 / 8.6 us, fp64 8.7 / 10.2 /
+// 17.7, fp64 2048^2 11.5 / 15.2 / 19.7.
+constexpr int kColWaves = 8;
+constexpr int kMinColsNarrow = 64;
 constexpr int kTargetBlocks = 2048;  // T form: blocks that keep HBM streaming
 
 int64_t imax(int64_t a, int64_t b) { return a > b ? a : b; }
@@ -59,12 +66,36 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 template <typename T>
 using vec4 = T __attribute__((ext_vector_type(4)));
+// The same four elements at element alignment: multi-dword global accesses
+// need dword alignment only, so any lda and base takes vector accesses.
+template <typename T>
+using vec4u = T __attribute__((ext_vector_type(4), aligned(sizeof(T))));
 
 // A is streamed once: non-temporal 4-element loads keep it from displacing x
 // and the partial sums in the caches.
 template <typename T>
 __device__ __forceinline__ vec4<T> ld_nt(const T *p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const vec4<T> *>(p));
+  return __builtin_nontemporal_load(reinterpret_cast<const vec4u<T> *>(p));
+}
+
+// How a kernel accesses A (its VEC parameter): kElems, fewer rows than a
+// vector; kVecU, vectors at element alignment; kVecA, vectors at their own
+// alignment (lda % 4 == 0 and A aligned to 4 elements), non-temporal. Neighbour
+// lanes' unaligned vectors share lines, which a non-temporal access fetches
+// again (ger 5001^2, lda 5002, non-temporal / not: fp32 47.7 / 36.7 us, fp64
+// 110 / 72; with element accesses 68.5 / 94.7).
+constexpr int kElems = 0, kVecU = 1, kVecA = 2;
+
+template <int VEC, typename T>
+__device__ __forceinline__ vec4<T> ld(const T *p) {
+  if constexpr (VEC == kVecA) return ld_nt(p);
+  return *reinterpret_cast<const vec4u<T> *>(p);
+}
+
+template <typename T>
+int access_of(int64_t rows, const T *A, int64_t lda) {
+  if (rows < 4) return kElems;
+  return lda % 4 == 0 && (uintptr_t)A % (4 * sizeof(T)) == 0 ? kVecA : kVecU;
 }
 
 // p aligned to 4 elements (the vector loads' alignment)
@@ -81,93 +112,92 @@ __device__ __forceinline__ void store_y(T *y, int64_t idx, T acc, T alpha, T bet
   y[idx] = v;
 }
 
-// N form. Block b, split s: columns [s*cps, min(n, (s+1)*cps)); rows in
-// kGroupsN groups of 1024, lane t of group g owning rows
-// [b*1024*kGroupsN + g*1024 + 4t, +4) (every load instruction of a wave
-// reads 256 elements of one column). VEC: lda % 4 == 0 and A aligned to 4
-// elements.
-template <typename T, bool VEC>
-__global__ __launch_bounds__(kThreads) void gemv_n_kernel(int64_t m, int64_t n,
-                                                          const T *__restrict__ A, int64_t lda,
-                                                          const T *__restrict__ x, int64_t incx,
-                                                          int64_t cps, T *__restrict__ part,
-                                                          T alpha, T beta,
-                                                          T *__restrict__ y, int64_t incy) {
+// N form. A block is RW x CW waves: RW of them side by side over the rows
+// (256 each, 4 consecutive rows per lane: every load instruction of a wave
+// reads 256 elements of one column), CW over the split's columns. Block b,
+// split s: rows [256 RW b, +256 RW), columns [s cps, min(n, (s+1) cps)), cps a
+// multiple of CW kStepN where CW > 1; the CW partial sums of a row are added through LDS in wave
+// order. VEC not kElems (m >= 4): a lane whose rows cross m (or lie past it) reads
+// the matrix's last 4 rows instead, in bounds, and stores only its own.
+template <typename T, int VEC, int RW, int CW>
+__global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t n,
+                                                              const T *__restrict__ A, int64_t lda,
+                                                              const T *__restrict__ x, int64_t incx,
+                                                              int64_t cps, T *__restrict__ part,
+                                                              T alpha, T beta,
+                                                              T *__restrict__ y, int64_t incy) {
   typedef vec4<T> f4;
-  constexpr int G = kGroupsN;
-  const int64_t rb = (int64_t)blockIdx.x * (4 * kThreads * G) + 4 * threadIdx.x;
-  const int64_t j0 = (int64_t)blockIdx.y * cps;
-  const int64_t j1 = j0 + cps < n ? j0 + cps : n;
-  if (rb >= m) return;
-  // rows past m read row m-1 (in bounds) and are never stored
-  int64_t ir[G][4];
-  bool full[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int64_t i0 = rb + (int64_t)g * 4 * kThreads;
-    full[g] = i0 + 4 <= m;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) ir[g][q] = i0 + q < m ? i0 + q : m - 1;
-  }
-  T acc[G][4];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[g][q] = (T)0;
-  auto load = [&](const T *col, int g) -> f4 {
-    if (VEC && full[g]) return ld_nt(col + ir[g][0]);
-    return f4{col[ir[g][0]], col[ir[g][1]], col[ir[g][2]], col[ir[g][3]]};
-  };
-  int64_t j = j0;
-  // kStepN columns per step, every load issued before the arithmetic
-  for (; j + kStepN <= j1; j += kStepN) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int rw = wave % RW, cw = wave / RW;
+  const int64_t rb = (int64_t)blockIdx.x * (256 * RW) + 256 * rw + 4 * lane;
+  // CW == 1: a lane with fewer than 4 rows reads them one by one instead (the
+  // per-lane branch keeps each step's loads together: 16384^2 161 us fp32, 333
+  // fp64, against 171 and 342 with the clamped vectors)
+  const bool whole = rb + 4 <= m;
+  if (CW == 1 && rb >= m) return;
+  const int64_t i0 = VEC && CW > 1 ? (rb <= m - 4 ? rb : m - 4) : (rb < m ? rb : 0);
+  int64_t j = (int64_t)blockIdx.y * cps;
+  int64_t j1 = j + cps < n ? j + cps : n;
+  j += cw * (cps / CW);
+  if (CW > 1 && j1 > j + cps / CW) j1 = j + cps / CW;
+  T acc[4] = {(T)0, (T)0, (T)0, (T)0};
+  // kStepN columns per step, every load issued before the arithmetic. LAST:
+  // columns past j1 repeat the last one against a zero x entry, which skips them
+  auto step = [&](auto last_tag) {
+    constexpr bool LAST = decltype(last_tag)::value;
     T xv[kStepN];
-    f4 av[kStepN][G];
+    f4 av[kStepN];
 #pragma unroll
-    for (int c = 0; c < kStepN; ++c) xv[c] = x[(j + c) * incx];
+    for (int c = 0; c < kStepN; ++c) {
+      const T v = x[(!LAST || j + c < j1 ? j + c : j1 - 1) * incx];
+      xv[c] = !LAST || j + c < j1 ? v : (T)0;
+    }
 #pragma unroll
-    for (int c = 0; c < kStepN; ++c)
+    for (int c = 0; c < kStepN; ++c) {
+      const T *col = A + (!LAST || j + c < j1 ? j + c : j1 - 1) * lda;
+      if (VEC && (CW > 1 || whole)) {
+        av[c] = ld<VEC>(col + i0);
+      } else {
 #pragma unroll
-      for (int g = 0; g < G; ++g) av[c][g] = load(A + (j + c) * lda, g);
+        for (int q = 0; q < 4; ++q) av[c][q] = col[i0 + q < m ? i0 + q : m - 1];
+      }
+    }
 #pragma unroll
     for (int c = 0; c < kStepN; ++c) {
       if (xv[c] != (T)0) {
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[g][q] = fma(av[c][g][q], xv[c], acc[g][q]);
+        for (int q = 0; q < 4; ++q) acc[q] = fma(av[c][q], xv[c], acc[q]);
       }
     }
-  }
-  for (; j < j1; ++j) {
-    const T xj = x[j * incx];
-    f4 a[G];
+  };
+  for (; j + kStepN <= j1; j += kStepN) step(std::false_type{});
+  if (j < j1) step(std::true_type{});
+  if constexpr (CW > 1) {
+    __shared__ T red[CW - 1][RW * 64][4];
+    if (cw > 0) {
 #pragma unroll
-    for (int g = 0; g < G; ++g) a[g] = load(A + j * lda, g);
-    if (xj != (T)0) {
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[g][q] = fma(a[g][q], xj, acc[g][q]);
+      for (int q = 0; q < 4; ++q) red[cw - 1][64 * rw + lane][q] = acc[q];
     }
+    __syncthreads();
+    if (cw > 0) return;
+#pragma unroll
+    for (int c = 0; c < CW - 1; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] += red[c][64 * rw + lane][q];
   }
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int64_t i0 = rb + (int64_t)g * 4 * kThreads;
-    const int rows = i0 >= m ? 0 : (full[g] ? 4 : (int)(m - i0));
-    for (int q = 0; q < rows; ++q) {
-      if (part)
-        part[(int64_t)blockIdx.y * m + i0 + q] = acc[g][q];
-      else
-        store_y(y, (i0 + q) * incy, acc[g][q], alpha, beta);
-    }
+  for (int q = 0; q < 4; ++q) {
+    const int64_t i = i0 + q;
+    if (i < rb || i >= m) continue;  // another lane's row, or none
+    if (part)
+      part[(int64_t)blockIdx.y * m + i] = acc[q];
+    else
+      store_y(y, i * incy, acc[q], alpha, beta);
   }
 }
 
 // T form. Wave w (4 per block) owns columns [CPW w, CPW w + CPW) of split s, rows
-// [s*rps, min(m, (s+1)*rps)). VEC: lda % 4 == 0, A 16-byte aligned, incx == 1
-// and x 16-byte aligned (rps is a multiple of 4, so every 4-row group of a
-// split starts aligned).
+// [s*rps, min(m, (s+1)*rps)). VEC: incx == 1 (A, lda and x at any alignment).
 template <typename T, bool VEC, int CPW>
 __global__ __launch_bounds__(kThreads) void gemv_t_kernel(int64_t m, int64_t n,
                                                           const T *__restrict__ A, int64_t lda,
@@ -192,8 +222,8 @@ __global__ __launch_bounds__(kThreads) void gemv_t_kernel(int64_t m, int64_t n,
   if (VEC) {
     // two 256-row groups per step: 16 loads of A in flight per lane
     for (; i + 256 + 4 <= r1; i += 512) {
-      const f4 xv0 = *reinterpret_cast<const f4 *>(x + i);
-      const f4 xv1 = *reinterpret_cast<const f4 *>(x + i + 256);
+      const f4 xv0 = *reinterpret_cast<const vec4u<T> *>(x + i);
+      const f4 xv1 = *reinterpret_cast<const vec4u<T> *>(x + i + 256);
       f4 av0[CPW], av1[CPW];
 #pragma unroll
       for (int c = 0; c < CPW; ++c) {
@@ -216,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void gemv_t_kernel(int64_t m, int64_t n,
   }
   for (; i < r1; i += 256) {
     if (VEC && i + 4 <= r1) {
-      const f4 xv = *reinterpret_cast<const f4 *>(x + i);
+      const f4 xv = *reinterpret_cast<const vec4u<T> *>(x + i);
       f4 av[CPW];
 #pragma unroll
       for (int c = 0; c < CPW; ++c) av[c] = ld_nt(col[c] + i);
@@ -837,19 +867,23 @@ int gemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, T alpha, const T *A, int
     wgb::timing_end(ctx);
     return WGB_OK;
   }
-  const bool vecA = lda % 4 == 0 && aligned4(A);
   // blocks along the output; split the contraction dimension until about
   // the target block count streams A (N: >= kMinColsN columns per split; T: >= 256
   // rows, a multiple of 256 so every split starts aligned)
   const int cpw = m <= kShortColsRows ? kColsPerWaveShort : kColsPerWave;  // T form
-  const int64_t bx = nt ? cdiv(m, 4 * kThreads * kGroupsN) : cdiv(cdiv(n, cpw), kThreads / 64);
+  // N form: where 1024-row blocks of at least kMinColsN columns are fewer than
+  // the target, blocks of 256 rows whose waves share the columns
+  const bool narrow = nt && cdiv(m, 4 * kThreads) * cdiv(n, kMinColsN) < kTargetBlocksN;
+  const int64_t bx = nt ? cdiv(m, narrow ? 256 : 4 * kThreads) : cdiv(cdiv(n, cpw), kThreads / 64);
   const int64_t target = nt ? kTargetBlocksN : kTargetBlocks;
   int64_t want = bx >= target ? 1 : cdiv(target, bx);
-  const int64_t most = nt ? cdiv(n, kMinColsN) : cdiv(m, 256);
+  const int64_t most = nt ? cdiv(n, narrow ? kMinColsNarrow : kMinColsN) : cdiv(m, 256);
   if (want > most) want = most;
   if (want > 65535) want = 65535;  // grid y limit
   if (want < 1) want = 1;
-  const int64_t per = nt ? cdiv(n, want) : cdiv(cdiv(m, want), 256) * 256;
+  // (narrow: whole steps for every wave)
+  const int64_t unit = narrow ? kColWaves * kStepN : 1;
+  const int64_t per = nt ? cdiv(cdiv(n, want), unit) * unit : cdiv(cdiv(m, want), 256) * 256;
   const int64_t splits = nt ? cdiv(n, per) : cdiv(m, per);
   T *part = nullptr;
   if (splits > 1) {
@@ -861,15 +895,23 @@ int gemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, T alpha, const T *A, int
   }
   dim3 grid((unsigned)bx, (unsigned)splits);
   if (nt) {
-    if (vecA)
-      gemv_n_kernel<T, true><<<grid, kThreads, 0, ctx->stream>>>(m, n, A, lda, x, incx, per, part,
-                                                               alpha, beta, y, incy);
+    const int vec = access_of(m, A, lda);
+    auto launch = [&](auto kern, int threads) {
+      kern<<<grid, threads, 0, ctx->stream>>>(m, n, A, lda, x, incx, per, part, alpha, beta, y, incy);
+    };
+    if (narrow)
+      launch(vec == kVecA   ? gemv_n_kernel<T, kVecA, 1, kColWaves>
+             : vec == kVecU ? gemv_n_kernel<T, kVecU, 1, kColWaves>
+                            : gemv_n_kernel<T, kElems, 1, kColWaves>,
+             64 * kColWaves);
     else
-      gemv_n_kernel<T, false><<<grid, kThreads, 0, ctx->stream>>>(m, n, A, lda, x, incx, per, part,
-                                                                alpha, beta, y, incy);
+      launch(vec == kVecA   ? gemv_n_kernel<T, kVecA, 4, 1>
+             : vec == kVecU ? gemv_n_kernel<T, kVecU, 4, 1>
+                            : gemv_n_kernel<T, kElems, 4, 1>,
+             kThreads);
     WGB_CHECK_LAUNCH("gemv_n_kernel");
   } else {
-    const bool vec = vecA && incx == 1 && aligned4(x);
+    const bool vec = incx == 1;
     auto launch = [&](auto kern) {
       kern<<<grid, kThreads, 0, ctx->stream>>>(m, n, A, lda, x, incx, per, part, alpha, beta, y, incy);
     };
