@@ -316,51 +316,86 @@ __global__ __launch_bounds__(kThreads) void scale_y_kernel(int64_t len, T beta, 
   if (i < len) y[i * incy] = beta == (T)0 ? (T)0 : beta * y[i * incy];
 }
 
+// Triangles of order n are walked as chunks of 1024 rows (4 consecutive rows
+// per lane of a block), each with the columns that its rows meet, kTriStep
+// columns at a time. All chunks' columns are laid end to end, each chunk's
+// count rounded up to whole steps, and cut into equal runs, one per block: a
+// rectangular grid over (chunk, panel) launches the other triangle's blocks
+// for nothing and leaves the last round of working ones uneven.
+constexpr int64_t kChunkRows = 4 * kThreads;
+constexpr int kTriStep = 8;
+
+// First column of chunk r (0 for a lower triangle, its first row for an upper
+// one) and the columns laid before and within it.
+template <bool LOWER>
+__host__ __device__ __forceinline__ int64_t chunk_first(int64_t r) {
+  return LOWER ? 0 : r * kChunkRows;
+}
+template <bool LOWER>
+__host__ __device__ __forceinline__ int64_t chunk_offset(int64_t n, int64_t r) {
+  const int64_t n8 = (n + kTriStep - 1) / kTriStep * kTriStep;
+  return LOWER ? kChunkRows * (r * (r + 1) / 2) : r * n8 - kChunkRows * (r * (r - 1) / 2);
+}
+template <bool LOWER>
+__host__ __device__ __forceinline__ int64_t chunk_columns(int64_t n, int64_t r) {
+  const int64_t n8 = (n + kTriStep - 1) / kTriStep * kTriStep;
+  return LOWER ? ((r + 1) * kChunkRows < n8 ? (r + 1) * kChunkRows : n8) : n8 - r * kChunkRows;
+}
+template <bool LOWER>
+int64_t triangle_columns(int64_t n) {
+  const int64_t last = (n - 1) / kChunkRows;
+  return chunk_offset<LOWER>(n, last) + chunk_columns<LOWER>(n, last);
+}
+
+// Calls body(r, c0, c1) for each chunk r of which block b's run, [b run,
+// (b + 1) run), holds columns [c0, c1).
+template <bool LOWER, class Body>
+__device__ __forceinline__ void walk_triangle(int64_t n, int64_t run, Body body) {
+  const int64_t f = (int64_t)blockIdx.x * run;
+  int64_t off = 0;
+  for (int64_t r = 0; r * kChunkRows < n && off < f + run; ++r) {
+    const int64_t cols = chunk_columns<LOWER>(n, r), first = chunk_first<LOWER>(r);
+    const int64_t a = f > off ? f - off : 0, b = f + run - off < cols ? f + run - off : cols;
+    if (a < b) body(r, first + a, first + b < n ? first + b : n);
+    off += cols;
+  }
+}
+
 // Rank-1 and rank-2 updates, A m x n column-major:
 //   ger  (UPLO 0, !TWO): A += alpha x y^T;
 //   syr  (UPLO 1 / 2, !TWO, y = x): the lower (i >= j) / upper (i <= j)
 //        triangle of A += alpha x x^T;
 //   syr2 (UPLO 1 / 2, TWO): that triangle of A += alpha x y^T + alpha y x^T.
-// Block (b, c): rows [1024 b, +1024) (4 consecutive rows per lane, its x
-// (and y) entries held in registers), columns [c cpb, min(n, (c+1) cpb)),
+// A block takes 1024 rows (4 consecutive ones per lane, its x (and y) entries
+// held in registers) of a run of columns: for ger, block (b, c) rows
+// [1024 b, +1024) and columns [c cpb, min(n, (c+1) cpb)); for a triangle, block
+// b its run of cpb of the chunks' columns (walk_triangle). Columns go
 // kStepG at a time with all of a step's A loads in flight. Column j takes
 // t1 = alpha y[j] (and t2 = alpha x[j]) and A(i, j) = fma(x[i], t1, A(i, j))
 // (then fma(y[i], t2, .)); a column whose y entry (for syr2: both entries)
 // is zero is neither computed nor written, reference BLAS's skip: Infinity or
 // NaN in the row vector never meets that zero. A is read and written once:
 // HBM-bound, 2 m n elements of traffic (half that for a triangle).
-constexpr int kStepG = 8;
-template <typename T, bool VEC, int UPLO, bool TWO>
+constexpr int kStepG = kTriStep;
+template <typename T, int VEC, int UPLO, bool TWO>
 __global__ __launch_bounds__(kThreads) void rank_update_kernel(
     int64_t m, int64_t n, T alpha, const T *__restrict__ x, int64_t incx, const T *__restrict__ y,
     int64_t incy, T *__restrict__ A, int64_t lda, int64_t cpb) {
   typedef vec4<T> f4;
-  const int64_t r0 = (int64_t)blockIdx.x * (4 * kThreads);
-  const int64_t i0 = r0 + 4 * threadIdx.x;
-  if (i0 >= m) return;
+  // columns [j0, j1) of the 1024 rows from r0 on
+  auto chunk = [&](const int64_t r0, int64_t j0, int64_t j1) {
+  const int64_t ib = r0 + 4 * threadIdx.x;  // the lane's own rows start here
+  if (ib >= m) return;
+  // VEC not kElems (m >= 4): a lane whose rows cross m takes the matrix's last 4 rows, in
+  // bounds, and stores only its own, [lo, 4) of them
+  const int64_t i0 = VEC && ib > m - 4 ? m - 4 : ib;
+  const int lo = (int)(ib - i0);
   const int rows = i0 + 4 <= m ? 4 : (int)(m - i0);
   f4 xv, yv;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     xv[q] = q < rows ? x[(i0 + q) * incx] : (T)0;
     yv[q] = TWO && q < rows ? y[(i0 + q) * incy] : (T)0;
-  }
-  int64_t j0 = (int64_t)blockIdx.y * cpb;
-  int64_t j1 = j0 + cpb < n ? j0 + cpb : n;
-  // triangle: the block's columns split into whole ones (every row of the
-  // block inside the triangle) and diagonal ones (rows masked per element)
-  const int64_t rlast = r0 + 4 * kThreads - 1;  // the block's last row
-  int64_t d0 = j0, d1 = j0;                     // diagonal columns [d0, d1)
-  if (UPLO == 1) {                              // lower: i >= j
-    if (j1 > rlast + 1) j1 = rlast + 1;
-    d0 = j0 > r0 + 1 ? j0 : r0 + 1;
-    d1 = j1;
-    if (d0 > d1) d0 = d1;
-  } else if (UPLO == 2) {  // upper: i <= j
-    if (j0 < r0) j0 = r0;
-    d0 = j0;
-    d1 = j1 < rlast ? j1 : rlast;
-    if (d1 < d0) d1 = d0;
   }
   // update of one column's 4 rows (masked rows keep their value)
   auto column_scalars = [&](int64_t j, T &t1, T &t2) -> bool {
@@ -377,19 +412,17 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
       if (TWO) a[q] = fma(yv[q], t2, a[q]);
     }
   };
-  // FULL: every row of the block inside m (a block-uniform choice): whole
-  // non-temporal vectors with no per-lane branch between them, a step's
-  // loads all issued together; otherwise element accesses with clamped rows.
-  // (A per-lane choice between the two, measured for ger at 16384^2 with
-  // 512 blocks on one box: fp32 5.0 against 5.5 TB/s.) MASK (the diagonal
-  // columns of a triangle): the same loads and arithmetic, and each lane
-  // stores only its rows inside the triangle (whole vectors where all four
-  // are).
+  // FULL: every row of the wave inside m (a wave-uniform choice): whole
+  // non-temporal vectors with no per-lane branch between the stores. The loads
+  // are whole vectors in either case (m >= 4), at any alignment of A and lda.
+  // MASK (the diagonal columns of a triangle): the same loads and arithmetic,
+  // and each lane stores only its rows inside the triangle (whole vectors
+  // where all four are).
   auto walk = [&](auto full_tag, auto mask_tag, int64_t ja, int64_t jb) {
     constexpr bool FULL = decltype(full_tag)::value;
     constexpr bool MASK = decltype(mask_tag)::value;
     auto load = [&](const T *col) -> f4 {
-      if constexpr (FULL) return ld_nt(col + i0);
+      if constexpr (VEC) return ld<FULL ? VEC : kVecU>(col + i0);
       f4 v;
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = col[i0 + (q < rows ? q : 0)];
@@ -397,19 +430,25 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
     };
     auto store = [&](T *col, const f4 &v, int64_t j) {
       if constexpr (MASK) {
-        const bool all = UPLO == 1 ? i0 >= j : i0 + rows - 1 <= j;
+        const bool all = lo == 0 && (UPLO == 1 ? i0 >= j : i0 + rows - 1 <= j);
         if (!all) {
-          for (int q = 0; q < rows; ++q) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
             const int64_t i = i0 + q;
-            if (UPLO == 1 ? i >= j : i <= j) col[i] = v[q];
+            if (q >= lo && q < rows && (UPLO == 1 ? i >= j : i <= j)) col[i] = v[q];
           }
           return;
         }
       }
-      if constexpr (FULL) {
-        __builtin_nontemporal_store(v, reinterpret_cast<f4 *>(col + i0));
+      if (FULL || (VEC && lo == 0)) {
+        if constexpr (FULL && VEC == kVecA)
+          __builtin_nontemporal_store(v, reinterpret_cast<vec4u<T> *>(col + i0));
+        else
+          *reinterpret_cast<vec4u<T> *>(col + i0) = v;
       } else {
-        for (int q = 0; q < rows; ++q) col[i0 + q] = v[q];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q >= lo && q < rows) col[i0 + q] = v[q];
       }
     };
     int64_t j = ja;
@@ -438,7 +477,9 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
       }
     }
   };
-  const bool whole_rows = VEC && rlast < m;
+  // a wave's choice: the one wave that crosses m is the only slow one
+  const int64_t w0 = r0 + 256 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the wave's 256 rows
+  const bool whole_rows = VEC && w0 + 256 <= m;
   auto walk_range = [&](auto mask_tag, int64_t ja, int64_t jb) {
     if (ja >= jb) return;
     if (whole_rows)
@@ -446,17 +487,25 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
     else
       walk(std::false_type{}, mask_tag, ja, jb);
   };
-  if (UPLO == 0) {
+  // columns wholly inside the triangle for these 256 rows, and diagonal ones
+  // (row i of column j is stored where i >= j (lower) or i <= j (upper))
+  const int64_t da = j0 > w0 ? j0 : w0, db = j1 < w0 + 256 ? j1 : w0 + 256;
+  if constexpr (UPLO == 0) {
     walk_range(std::false_type{}, j0, j1);
-    return;
+  } else if constexpr (UPLO == 1) {
+    walk_range(std::false_type{}, j0, j1 < w0 ? j1 : w0);
+    walk_range(std::true_type{}, da, db);
+  } else {
+    walk_range(std::true_type{}, da, db);
+    walk_range(std::false_type{}, j0 > w0 + 256 ? j0 : w0 + 256, j1);
   }
-  // whole columns, then the diagonal ones: row i of column j is stored
-  // where i >= j (lower) or i <= j (upper)
-  if (UPLO == 1)
-    walk_range(std::false_type{}, j0, d0);
-  else
-    walk_range(std::false_type{}, d1, j1);
-  walk_range(std::true_type{}, d0, d1);
+  };
+  if constexpr (UPLO == 0) {
+    const int64_t j0 = (int64_t)blockIdx.y * cpb;
+    chunk((int64_t)blockIdx.x * kChunkRows, j0, j0 + cpb < n ? j0 + cpb : n);
+  } else {
+    walk_triangle<UPLO == 1>(n, cpb, [&](int64_t r, int64_t c0, int64_t c1) { chunk(r * kChunkRows, c0, c1); });
+  }
 }
 
 // ger (uplo 0, y given), syr (uplo 1 / 2, y == x, !two), syr2 (uplo 1 / 2,
@@ -480,33 +529,44 @@ int rank_update(wgb_ctx *ctx, int uplo, bool two, int64_t m, int64_t n, T alpha,
   // column chunks: about one block per CU in all for ger (each a long run of
   // columns), at least kStepG columns each. Measured at 16384^2 on one box,
   // blocks in all against TB/s (fp32 / fp64): 128 3.5 / 3.7, 256 5.7 / 5.2,
-  // 384 5.7 / 4.1, 512 5.5 / 4.9, 2048 4.8 / 4.7. A triangle's blocks do
-  // work that varies with their row; for fp32, four times as many, shorter
-  // blocks even it out (lower 16384, blocks per CU 1 / 2 / 4 / 8 / 16: ssyr
-  // 2.4 / 3.4 / 3.5 / 3.6 / 3.3 TB/s), fp64 kept one per CU (dsyr 3.4 / 3.0 /
-  // 3.1 / 3.1 / 3.2).
+  // 384 5.7 / 4.1, 512 5.5 / 4.9, 2048 4.8 / 4.7. Triangles: equal runs, two
+  // per CU for fp32 and one for fp64 (lower, 1 / 2 / 4 runs per CU: ssyr2 8192
+  // 63.7 / 52.9 / 52.9 us, 16384 211 / 207 / 205; dsyr2 8192 115 / 117 / 128,
+  // 16384 453 / 479 / 484; a rectangular grid took 80, 300, 200 and 632).
   const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  const int64_t target = uplo == 0 || sizeof(T) == 8 ? cus : 4 * cus;
-  int64_t chunks = cdiv(target, bx);
-  if (chunks > cdiv(n, kStepG)) chunks = cdiv(n, kStepG);
-  if (chunks > 65535) chunks = 65535;
-  if (chunks < 1) chunks = 1;
-  const int64_t cpb = cdiv(n, chunks);
-  const dim3 grid((unsigned)bx, (unsigned)cdiv(n, cpb));
-  const bool vec = lda % 4 == 0 && aligned4(A);
+  dim3 grid;
+  int64_t cpb;
+  if (uplo == 0) {
+    int64_t chunks = cdiv(cus, bx);
+    if (chunks > cdiv(n, kStepG)) chunks = cdiv(n, kStepG);
+    if (chunks > 65535) chunks = 65535;
+    if (chunks < 1) chunks = 1;
+    cpb = cdiv(n, chunks);
+    grid = dim3((unsigned)bx, (unsigned)cdiv(n, cpb));
+  } else {
+    const int64_t total = uplo == WGB_LOWER ? triangle_columns<true>(n) : triangle_columns<false>(n);
+    cpb = cdiv(cdiv(total, (sizeof(T) == 4 ? 2 : 1) * cus), kStepG) * kStepG;
+    grid = dim3((unsigned)cdiv(total, cpb));
+  }
   auto launch = [&](auto kern) {
     kern<<<grid, kThreads, 0, ctx->stream>>>(m, n, alpha, x, incx, y, incy, A, lda, cpb);
   };
-  if (uplo == 0)
-    launch(vec ? rank_update_kernel<T, true, 0, false> : rank_update_kernel<T, false, 0, false>);
-  else if (uplo == WGB_LOWER && !two)
-    launch(vec ? rank_update_kernel<T, true, 1, false> : rank_update_kernel<T, false, 1, false>);
-  else if (!two)
-    launch(vec ? rank_update_kernel<T, true, 2, false> : rank_update_kernel<T, false, 2, false>);
-  else if (uplo == WGB_LOWER)
-    launch(vec ? rank_update_kernel<T, true, 1, true> : rank_update_kernel<T, false, 1, true>);
+  auto by_form = [&](auto vec_tag) {
+    constexpr int VEC = decltype(vec_tag)::value;
+    if (uplo == 0)
+      launch(rank_update_kernel<T, VEC, 0, false>);
+    else if (uplo == WGB_LOWER)
+      launch(two ? rank_update_kernel<T, VEC, 1, true> : rank_update_kernel<T, VEC, 1, false>);
+    else
+      launch(two ? rank_update_kernel<T, VEC, 2, true> : rank_update_kernel<T, VEC, 2, false>);
+  };
+  const int vec = access_of(m, A, lda);
+  if (vec == kVecA)
+    by_form(std::integral_constant<int, kVecA>{});
+  else if (vec == kVecU)
+    by_form(std::integral_constant<int, kVecU>{});
   else
-    launch(vec ? rank_update_kernel<T, true, 2, true> : rank_update_kernel<T, false, 2, true>);
+    by_form(std::integral_constant<int, kElems>{});
   WGB_CHECK_LAUNCH("rank_update_kernel");
   wgb::timing_end(ctx);
   return WGB_OK;
