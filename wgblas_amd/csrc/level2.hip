@@ -98,12 +98,6 @@ int access_of(int64_t rows, const T *A, int64_t lda) {
   return lda % 4 == 0 && (uintptr_t)A % (4 * sizeof(T)) == 0 ? kVecA : kVecU;
 }
 
-// p aligned to 4 elements (the vector loads' alignment)
-template <typename T>
-bool aligned4(const T *p) {
-  return ((uintptr_t)p % (4 * sizeof(T))) == 0;
-}
-
 // Writes one output element: alpha * acc + beta * y (beta == 0 never reads y).
 template <typename T>
 __device__ __forceinline__ void store_y(T *y, int64_t idx, T acc, T alpha, T beta) {
@@ -573,78 +567,155 @@ int rank_update(wgb_ctx *ctx, int uplo, bool two, int64_t m, int64_t n, T alpha,
 }
 
 // ssymv / dsymv: y <- alpha S x + beta y, S the n x n symmetric matrix whose
-// uplo triangle A holds (column-major). The triangle is read once: block
-// (r, p) takes rows [1024 r, +1024) (4 per lane in each row group, their x
-// entries in registers) and panel p, columns [128 p, +128), 8 at a time with all of a
-// step's loads in flight, and uses each stored element twice: A(i, j) x(j)
-// for row i and, off the diagonal, A(i, j) x(i) for its mirror, row j. The
-// row sums of a panel go to rowpart[p][i]; the mirror sums of a column are
-// folded across each wave (shuffles) and, once at the end of the block,
-// across its 4 waves (LDS) into colpart[r][j]. symv_fold_kernel then adds, for each j, exactly the slots
-// the triangle's blocks wrote, in a fixed order (deterministic), and applies
-// alpha and beta. Every term is taken (no zero skipping, as reference BLAS's
-// symv). Blocks that cross the diagonal mask elements outside the triangle
-// by selecting their terms away (never multiplying them).
-// Measured at 16384 / 8192 (lower, TB/s of triangle traffic, fp32 / fp64):
-// 1 row group and 128-column panels 3.5 / 3.1 and 2.1 / 2.7; 2 groups 2.8 /
-// 2.9 and 1.4 / 1.8, 4 groups (4 columns a step) 2.7 / 2.3 and 0.8 / 1.0
-// (fewer blocks); 64-column panels 3.3 / 3.0 and 2.5 / 2.6, 32-column 3.2 /
-// 2.8 and 2.4 / 2.5.
-constexpr int kSymvGroups = 1;                         // 1024-row groups per block
-constexpr int kSymvRows = kSymvGroups * 4 * kThreads;  // rows per block
-constexpr int kSymvPanel = 128;                        // columns per block
-constexpr int kSymvStep = 8;                           // columns per step
+// uplo triangle A holds (column-major). The triangle is read once: a block
+// takes a run of columns of a chunk of 1024 rows (walk_triangle; 4 rows per
+// lane, their x entries in registers), 8 columns at a time with all of a
+// step's loads in flight, and uses each stored element twice: A(i, j) x(j) for
+// row i and, off the diagonal, A(i, j) x(i) for its mirror, row j. The row
+// sums of block b over chunk r go to row slot b - (r's first block)
+// (part[slot n + i]); the mirror sums of a column are folded across each wave
+// (fold8) and, once at the end of the run, across the 4 waves (LDS) into column
+// slot r (part[(slots + r) n + j]). symv_fold_kernel then adds, for each j,
+// exactly the slots that were written for it, in a fixed order (deterministic),
+// and applies alpha and beta. Every term is taken (no zero skipping, as
+// reference BLAS's symv). Waves that cross the diagonal mask elements outside
+// the triangle by selecting their terms away (never multiplying them).
+// HBM-bound: the triangle once. Lower, rectangular 1024 x 128 blocks with a
+// shuffle fold per column -> this: ssymv 16384 144 -> 89 us (6.0 TB/s), 8192 58
+// -> 28, 4096 50 -> 13; dsymv 16384 339 -> 192 (5.6 TB/s), 4096 65 -> 21.
+constexpr int kRunMax = 512;  // columns per block (the LDS of their sums)
+constexpr int kRunMin = 32;
+constexpr int64_t kSymvMaxN = (int64_t)65535 * 128;  // accepted orders
+constexpr int kSymvStep = kTriStep;                  // columns per step
+constexpr int kSymvFoldWaves = 8;
+
+// Columns per block, blocks, and row slots (the most blocks that meet one
+// chunk): equal runs, two per CU where they have kRunMin columns, and no more
+// than kRunMax allows (lower, 1 / 2 / 4 per CU: ssymv 8192 29.3 / 27.7 / 29.3
+// us, dsymv 8192 57.9 / 55.6 / 73.0, 16384 193 / 192 / 242; dsymv 4096, where
+// two would be 20 columns, 21.2 against 27.0 in runs of 32).
+struct SymvPlan {
+  int64_t run, blocks, slots;
+};
+template <bool LOWER>
+SymvPlan symv_plan(int64_t n, int64_t cus) {
+  const int64_t total = triangle_columns<LOWER>(n);
+  int64_t rounds = cdiv(total, cus * kRunMax);
+  if (rounds < 2) rounds = total >= 2 * cus * kRunMin ? 2 : 1;
+  int64_t run = cdiv(cdiv(total, rounds * cus), kTriStep) * kTriStep;
+  if (run < kRunMin) run = kRunMin;
+  SymvPlan p = {run, cdiv(total, run), 0};
+  for (int64_t r = 0; r * kChunkRows < n; ++r) {
+    const int64_t off = chunk_offset<LOWER>(n, r);
+    const int64_t meet = (off + chunk_columns<LOWER>(n, r) - 1) / run - off / run + 1;
+    if (meet > p.slots) p.slots = meet;
+  }
+  return p;
+}
+
+// Value of lane ^ 1, ^ 2 (quads), the mirror in 8 lanes, lane ^ 8: DPP moves,
+// one VALU instruction each (two for 8-byte values).
+template <int CTRL, typename T>
+__device__ __forceinline__ T dpp(T v) {
+  constexpr int W = sizeof(T) / 4;
+  int w[W];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (int k = 0; k < W; ++k) w[k] = __builtin_amdgcn_mov_dpp(w[k], CTRL, 0xf, 0xf, true);
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor8 = 0x128;
+
+// permlane32_swap exchanges a's upper 32 lanes with b's lower 32, so that the
+// two results' sum holds a's fold in the lower half and b's in the upper one;
+// permlane16_swap does the same with odd and even rows of 16 lanes.
+template <bool HALVES, typename T>
+__device__ __forceinline__ T swap_add(T a, T b) {
+  constexpr int W = sizeof(T) / 4;
+  unsigned wa[W], wb[W];
+  __builtin_memcpy(wa, &a, sizeof(T));
+  __builtin_memcpy(wb, &b, sizeof(T));
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    if constexpr (HALVES) {
+      const auto r = __builtin_amdgcn_permlane32_swap(wa[k], wb[k], false, false);
+      wa[k] = r[0];
+      wb[k] = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(wa[k], wb[k], false, false);
+      wa[k] = r[0];
+      wb[k] = r[1];
+    }
+  }
+  __builtin_memcpy(&a, wa, sizeof(T));
+  __builtin_memcpy(&b, wb, sizeof(T));
+  return a + b;
+}
+
+// Folds 8 values per lane over the wave: returns, in every lane, the sum of
+// v[lane / 8] over all 64 lanes. Each exchange halves the values a lane
+// still carries: 6 swaps and 4 DPP moves, against 48 LDS-routed shuffles for
+// 8 folds of their own.
+template <typename T>
+__device__ __forceinline__ T fold8(const T (&v)[8], int lane) {
+  T a[4], b[2];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) a[c] = swap_add<true>(v[c], v[c + 4]);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) b[c] = swap_add<false>(a[c], a[c + 2]);
+  const bool odd = lane & 8;
+  T s = (odd ? b[1] : b[0]) + dpp<kDppRor8>(odd ? b[0] : b[1]);
+  s += dpp<kDppXor1>(s);
+  s += dpp<kDppXor2>(s);
+  return s + dpp<kDppHalfMirror>(s);
+}
+
 // MODE 0: symv (row and mirror sums); 1: strmv without transpose (row sums
 // over the triangle, diagonal included, a column skipped where x is zero);
 // 2: strmv transposed (column sums over the triangle, diagonal included, no
 // skipping). UNIT: the diagonal taken as 1, its stored value never used.
-template <typename T, bool VEC, int UPLO, int MODE = 0, bool UNIT = false>
-__global__ __launch_bounds__(kThreads) void symv_kernel(int64_t n, const T *__restrict__ A, int64_t lda,
+// VEC not kElems (n >= 4): a lane whose rows cross n (or lie past it) reads the
+// matrix's last 4 rows, in bounds, and uses only its own.
+template <typename T, int VEC, int UPLO, int MODE = 0, bool UNIT = false>
+__global__ __launch_bounds__(kThreads) void symv_kernel(int64_t n, int64_t run, int64_t slots,
+                                                        const T *__restrict__ A, int64_t lda,
                                                         const T *__restrict__ x, int64_t incx,
-                                                        T *__restrict__ rowpart,
-                                                        T *__restrict__ colpart) {
+                                                        T *__restrict__ part) {
   typedef vec4<T> f4;
-  constexpr int G = kSymvGroups, S = kSymvStep;
-  const int64_t r0 = (int64_t)blockIdx.x * kSymvRows;
-  const int64_t c0 = (int64_t)blockIdx.y * kSymvPanel;
-  const int64_t rlast = r0 + kSymvRows - 1;
-  // does the block hold any element of the triangle? (block-uniform)
-  if (UPLO == 1 ? rlast < c0 : r0 > c0 + kSymvPanel - 1) return;
-  const int64_t cend = c0 + kSymvPanel < n ? c0 + kSymvPanel : n;
-  // a block strictly below (lower) / above (upper) the diagonal needs no
-  // masks: every element stored, none on the diagonal
-  const bool cross = UPLO == 1 ? r0 < cend : rlast >= c0;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool whole = VEC && rlast < n;  // every lane's rows inside n
-  // group g: this lane's 4 rows i0[g] .. i0[g]+3 (rows[g] of them inside n)
-  int64_t i0[G], ib[G];
-  int rows[G];
-  f4 xv[G];
-  T racc[G][4];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    i0[g] = r0 + (int64_t)g * 4 * kThreads + 4 * threadIdx.x;
-    rows[g] = i0[g] >= n ? 0 : (i0[g] + 4 <= n ? 4 : (int)(n - i0[g]));
-    ib[g] = rows[g] > 0 ? i0[g] : 0;  // a row inside the matrix
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      xv[g][q] = q < rows[g] ? x[(i0[g] + q) * incx] : (T)0;
-      racc[g][q] = (T)0;
-    }
-  }
+  constexpr int S = kSymvStep;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // per-wave column sums of every step, added across the waves once at the
   // end: no barrier between steps, so a step's loads never wait on the
   // previous step's reduction
-  __shared__ T red[kSymvPanel / S][4][S];
-  // the step loop, compiled once per (WHOLE, CROSS): with either as a
-  // run-time test the loads sat in separate branches and issued one by one
-  auto steps = [&](auto whole_tag, auto cross_tag) {
+  __shared__ T red[MODE == 1 ? 1 : kRunMax / S][4][S];
+  walk_triangle<UPLO == 1>(n, run, [&](const int64_t r, const int64_t c0, const int64_t cend) {
+  const int64_t r0 = r * kChunkRows;
+  const int64_t w0 = r0 + 256 * wave;  // the wave's 256 rows
+  const int64_t ib = r0 + 4 * threadIdx.x;  // this lane's rows: those of i0 .. i0 + 3 in [ib, n)
+  const int64_t i0 = VEC ? (ib <= n - 4 ? ib : n - 4) : (ib < n ? ib : 0);
+  f4 xv;
+  T racc[4];
+  bool own[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    own[q] = i0 + q >= ib && i0 + q < n;
+    xv[q] = own[q] ? x[(i0 + q) * incx] : (T)0;
+    racc[q] = (T)0;
+  }
+  // columns [ja, jb), a whole number of steps from c0 on. WHOLE: whole steps,
+  // and every lane's rows inside n or (PART) rows of other lanes taken as 0;
+  // CROSS: some element outside the triangle or on the diagonal. Compiled once
+  // per form: with any as a run-time test the loads sat in separate branches
+  // and issued one by one.
+  auto steps = [&](auto whole_tag, auto cross_tag, auto part_tag, int64_t ja, int64_t jb) {
     constexpr bool WHOLE = decltype(whole_tag)::value;
+    constexpr bool PART = decltype(part_tag)::value;
     constexpr bool CROSS = decltype(cross_tag)::value;
-    int step = 0;
-    for (int64_t j = c0; j < cend; j += S, ++step) {
-      const int cols = cend - j < S ? (int)(cend - j) : S;
-      f4 a[S][G];
+    int step = (int)(ja - c0) / S;
+    for (int64_t j = ja; j < jb; j += S, ++step) {
+      const int cols = WHOLE || jb - j >= S ? S : (int)(jb - j);
+      f4 a[S];
       T xc[S];
 #pragma unroll
       for (int c = 0; c < S; ++c) {
@@ -652,114 +723,133 @@ __global__ __launch_bounds__(kThreads) void symv_kernel(int64_t n, const T *__re
         const T xj = x[jc * incx];
         xc[c] = c < cols ? xj : (T)0;
         const T *col = A + jc * lda;
+        if constexpr (VEC) {
+          a[c] = ld<VEC>(col + i0);
+        } else {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-          if constexpr (WHOLE) {
-            a[c][g] = ld_nt(col + i0[g]);
-          } else {
-            // rows past n read row ib (inside the matrix) and are never
-            // used; a lane with no rows in a group (kept for the block's
-            // final barrier) reads row 0
-#pragma unroll
-            for (int q = 0; q < 4; ++q) a[c][g][q] = col[ib[g] + (q < rows[g] ? q : 0)];
-          }
+          for (int q = 0; q < 4; ++q) a[c][q] = col[i0 + q < n ? i0 + q : n - 1];
         }
       }
       T cacc[S];
+      T rstep[4] = {(T)0, (T)0, (T)0, (T)0};  // the step's row sums: a chain of 8 products, then one add
+      const int d = CROSS ? (int)(i0 - j) : 0;
 #pragma unroll
       for (int c = 0; c < S; ++c) {
         cacc[c] = (T)0;
-        const int64_t jc = j + c;
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int64_t i = i0[g] + q;
-            bool in = c < cols && q < rows[g];  // stored element (i, jc)
-            bool mirror = in;                   // ... off the diagonal
-            if constexpr (CROSS) {
-              in = in && (UPLO == 1 ? i >= jc : i <= jc);
-              mirror = in && i != jc;
-            }
-            T av = a[c][g][q];
-            if constexpr (UNIT && CROSS) av = i == jc ? (T)1 : av;  // only a crossing block holds the diagonal
-            if constexpr (MODE == 0) {
-              racc[g][q] = in ? fma(av, xc[c], racc[g][q]) : racc[g][q];
-              cacc[c] = mirror ? fma(av, xv[g][q], cacc[c]) : cacc[c];
-            } else if constexpr (MODE == 1) {
-              // reference BLAS's column form: a zero x entry skips its column
-              racc[g][q] = in && xc[c] != (T)0 ? fma(av, xc[c], racc[g][q]) : racc[g][q];
-            } else {
-              cacc[c] = in ? fma(av, xv[g][q], cacc[c]) : cacc[c];
-            }
+        for (int q = 0; q < 4; ++q) {
+          bool in = WHOLE || (c < cols && own[q]);  // stored element (i0 + q, j + c) of this lane
+          bool mirror = in;                         // ... off the diagonal
+          if constexpr (CROSS) {
+            in = in && (UPLO == 1 ? d >= c - q : d <= c - q);
+            mirror = in && d != c - q;
+          }
+          T av = a[c][q];
+          if constexpr (PART) av = own[q] ? av : (T)0;
+          if constexpr (UNIT && CROSS) av = d == c - q ? (T)1 : av;  // only a crossing block holds the diagonal
+          if constexpr (MODE == 0) {
+            rstep[q] = in ? fma(av, xc[c], rstep[q]) : rstep[q];
+            cacc[c] = mirror ? fma(av, xv[q], cacc[c]) : cacc[c];
+          } else if constexpr (MODE == 1) {
+            // reference BLAS's column form: a zero x entry skips its column
+            rstep[q] = in && xc[c] != (T)0 ? fma(av, xc[c], rstep[q]) : rstep[q];
+          } else {
+            cacc[c] = in ? fma(av, xv[q], cacc[c]) : cacc[c];
           }
         }
       }
-      if constexpr (MODE == 1) continue;  // row sums only
-      // the step's column sums across the wave
+      if constexpr (MODE != 2) {
 #pragma unroll
-      for (int c = 0; c < S; ++c) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) cacc[c] += __shfl_xor(cacc[c], off, 64);
+        for (int q = 0; q < 4; ++q) racc[q] += rstep[q];
       }
-      if (lane < S) {
-        T v = cacc[0];
-#pragma unroll
-        for (int c = 1; c < S; ++c) v = lane == c ? cacc[c] : v;
-        red[step][wave][lane] = v;
+      if constexpr (MODE != 1) {  // the step's column sums across the wave
+        const T v = fold8(cacc, lane);
+        if ((lane & 7) == 0) red[step][wave][lane >> 3] = v;
       }
     }
   };
-  if (whole && !cross)
-    steps(std::true_type{}, std::false_type{});
-  else if (whole)
-    steps(std::true_type{}, std::true_type{});
-  else
-    steps(std::false_type{}, std::true_type{});
+  auto range = [&](auto cross_tag, int64_t ja, int64_t jb) {
+    if (ja >= jb) return;
+    const bool all = w0 + 256 <= n;
+    const int64_t jw = VEC && (all || !decltype(cross_tag)::value) ? ja + (jb - ja) / S * S : ja;
+    if (ja < jw) {
+      if (all)
+        steps(std::true_type{}, cross_tag, std::false_type{}, ja, jw);
+      else if constexpr (!decltype(cross_tag)::value)
+        steps(std::true_type{}, cross_tag, std::true_type{}, ja, jw);
+    }
+    if (jw < jb) steps(std::false_type{}, std::true_type{}, std::false_type{}, jw, jb);
+  };
+  // for the wave's 256 rows: columns all inside the triangle and off the
+  // diagonal, columns that cross it, and columns outside (their sums are 0)
+  const int64_t lo = c0 > w0 ? c0 : w0, hi = cend < w0 + 256 ? cend : w0 + 256;
+  if constexpr (UPLO == 1) {
+    if (w0 < n) {
+      range(std::false_type{}, c0, cend < w0 ? cend : w0);
+      range(std::true_type{}, lo, hi);
+    }
+  } else {
+    range(std::true_type{}, lo, hi);
+    range(std::false_type{}, c0 > w0 + 256 ? c0 : w0 + 256, cend);
+  }
+  if constexpr (MODE != 1) {
+    const int64_t za = UPLO == 1 && w0 < n ? (c0 > w0 + 256 ? c0 : w0 + 256) : c0;
+    const int64_t zb = UPLO == 1 ? cend : (cend < w0 ? cend : w0);
+    for (int64_t j = za + lane; j < zb; j += 64) red[(j - c0) / S][wave][(j - c0) % S] = (T)0;
+  }
   if (MODE != 2) {
+    const int64_t slot = (int64_t)blockIdx.x - chunk_offset<UPLO == 1>(n, r) / run;
 #pragma unroll
-    for (int g = 0; g < G; ++g)
-      for (int q = 0; q < rows[g]; ++q) rowpart[(int64_t)blockIdx.y * n + i0[g] + q] = racc[g][q];
+    for (int q = 0; q < 4; ++q)
+      if (own[q]) part[slot * n + i0 + q] = racc[q];
   }
-  if (MODE == 1) return;  // uniform, after the last use of red
-  __syncthreads();
-  if (threadIdx.x < cend - c0) {
-    const int st = threadIdx.x / S, c = threadIdx.x % S;
-    const T v = ((red[st][0][c] + red[st][1][c]) + red[st][2][c]) + red[st][3][c];
-    colpart[(int64_t)blockIdx.x * n + c0 + threadIdx.x] = v;
+  if constexpr (MODE != 1) {
+    __syncthreads();
+    T *colpart = part + (slots + r) * n + c0;
+    for (int t = threadIdx.x; t < cend - c0; t += kThreads) {
+      const int st = t / S, c = t % S;
+      colpart[t] = ((red[st][0][c] + red[st][1][c]) + red[st][2][c]) + red[st][3][c];
+    }
+    __syncthreads();  // the next chunk's sums take the same LDS
   }
+  });
 }
 
-// y(j) <- alpha (sum of the row sums of the panels that reach row j + sum of
-// the mirror sums of the row chunks that reach column j) + beta y(j): the
-// slots symv_kernel wrote for j, lower (UPLO 1): panels 0 .. j/128, chunks
-// from the one holding row 128 (j/128) on; upper: panels j/128 .. P-1, chunks
-// up to the one holding row 128 (j/128) + 127. beta == 0 never reads y.
+// y(j) <- alpha (sum of the row slots of j's chunk + sum of the column slots of
+// the chunks that meet column j) + beta y(j). A block folds 64 outputs (one
+// chunk's): its waves take 8 slots at a time in turn, added in wave order
+// through LDS. beta == 0 never reads y.
 template <typename T, int UPLO, int MODE = 0>
-__global__ __launch_bounds__(kThreads) void symv_fold_kernel(int64_t n, const T *__restrict__ rowpart,
-                                                             const T *__restrict__ colpart, T alpha,
-                                                             T beta, T *__restrict__ y, int64_t incy) {
-  const int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (j >= n) return;
-  const int64_t np = (n + kSymvPanel - 1) / kSymvPanel, nr = (n + kSymvRows - 1) / kSymvRows;
-  const int64_t pj = j / kSymvPanel;
-  const int64_t p0 = UPLO == 1 ? 0 : pj, p1 = UPLO == 1 ? pj + 1 : np;
-  const int64_t ra = UPLO == 1 ? (pj * kSymvPanel) / kSymvRows : 0;
-  const int64_t rb = UPLO == 1 ? nr : (pj * kSymvPanel + kSymvPanel - 1) / kSymvRows + 1;
+__global__ __launch_bounds__(64 * kSymvFoldWaves) void symv_fold_kernel(int64_t n, int64_t run, int64_t slots,
+                                                                        const T *__restrict__ part, T alpha,
+                                                                        T beta, T *__restrict__ y, int64_t incy) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t j = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t jl = j < n ? j : n - 1;  // lanes past n fold column n - 1 and store nothing
+  const int64_t r = (int64_t)blockIdx.x * 64 / kChunkRows, nr = (n + kChunkRows - 1) / kChunkRows;
+  const int64_t off = chunk_offset<UPLO == 1>(n, r);
+  // row sums (symv, strmv without transpose), then column sums (symv's
+  // mirrors, strmv transposed)
+  const int rows = MODE != 2 ? (int)((off + chunk_columns<UPLO == 1>(n, r) - 1) / run - off / run + 1) : 0;
+  const int64_t ra = UPLO == 1 ? r : 0;
+  const int total = rows + (MODE != 1 ? (int)((UPLO == 1 ? nr : r + 1) - ra) : 0);
   T s = (T)0;
-  if (MODE != 2) {  // row sums (symv, strmv without transpose)
-    int64_t p = p0;
-    for (; p + 8 <= p1; p += 8) {
-      T v[8];
+  for (int k = 8 * wave; k < total; k += 8 * kSymvFoldWaves) {
+    T v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = rowpart[(p + u) * n + j];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
+    for (int u = 0; u < 8; ++u) {
+      const int q = k + u < total ? k + u : total - 1;
+      v[u] = part[(q < rows ? q : slots + ra + q - rows) * n + jl];
     }
-    for (; p < p1; ++p) s += rowpart[p * n + j];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s = k + u < total ? s + v[u] : s;
   }
-  if (MODE != 1)  // column sums (symv's mirrors, strmv transposed)
-    for (int64_t r = ra; r < (rb < nr ? rb : nr); ++r) s += colpart[r * n + j];
+  __shared__ T red[kSymvFoldWaves][64];
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave > 0 || j >= n) return;
+#pragma unroll
+  for (int w = 1; w < kSymvFoldWaves; ++w) s += red[w][lane];
   T v = alpha * s;
   if (beta != (T)0) v = fma(beta, y[j * incy], v);
   y[j * incy] = v;
@@ -793,27 +883,27 @@ int symv(wgb_ctx *ctx, int uplo, int64_t n, T alpha, const T *A, int64_t lda, co
     wgb::timing_end(ctx);
     return WGB_OK;
   }
-  const int64_t nr = cdiv(n, kSymvRows), np = cdiv(n, kSymvPanel);
-  if (np > 65535) return fail(WGB_ERR_INVALID_VALUE, "n too large for one launch");
-  if ((st = wgb::ensure_op_workspace(ctx, (size_t)((np + nr) * n) * sizeof(T)))) return st;
-  T *rowpart = static_cast<T *>(ctx->op_ws);
-  T *colpart = rowpart + np * n;
-  const dim3 grid((unsigned)nr, (unsigned)np);
-  const bool vec = lda % 4 == 0 && aligned4(A);
-  auto launch = [&](auto kern) {
-    kern<<<grid, kThreads, 0, ctx->stream>>>(n, A, lda, x, incx, rowpart, colpart);
+  if (n > kSymvMaxN) return fail(WGB_ERR_INVALID_VALUE, "n too large for one launch");
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const SymvPlan plan = uplo == WGB_LOWER ? symv_plan<true>(n, cus) : symv_plan<false>(n, cus);
+  if ((st = wgb::ensure_op_workspace(ctx, (size_t)((plan.slots + cdiv(n, kChunkRows)) * n) * sizeof(T)))) return st;
+  T *part = static_cast<T *>(ctx->op_ws);
+  auto launch = [&](auto vec_tag) {
+    constexpr int VEC = decltype(vec_tag)::value;
+    auto kern = uplo == WGB_LOWER ? symv_kernel<T, VEC, 1> : symv_kernel<T, VEC, 2>;
+    kern<<<(unsigned)plan.blocks, kThreads, 0, ctx->stream>>>(n, plan.run, plan.slots, A, lda, x, incx, part);
   };
-  if (uplo == WGB_LOWER)
-    launch(vec ? symv_kernel<T, true, 1> : symv_kernel<T, false, 1>);
+  const int vec = access_of(n, A, lda);
+  if (vec == kVecA)
+    launch(std::integral_constant<int, kVecA>{});
+  else if (vec == kVecU)
+    launch(std::integral_constant<int, kVecU>{});
   else
-    launch(vec ? symv_kernel<T, true, 2> : symv_kernel<T, false, 2>);
+    launch(std::integral_constant<int, kElems>{});
   WGB_CHECK_LAUNCH("symv_kernel");
-  if (uplo == WGB_LOWER)
-    symv_fold_kernel<T, 1><<<(unsigned)cdiv(n, kThreads), kThreads, 0, ctx->stream>>>(
-        n, rowpart, colpart, alpha, beta, y, incy);
-  else
-    symv_fold_kernel<T, 2><<<(unsigned)cdiv(n, kThreads), kThreads, 0, ctx->stream>>>(
-        n, rowpart, colpart, alpha, beta, y, incy);
+  auto fold = uplo == WGB_LOWER ? symv_fold_kernel<T, 1> : symv_fold_kernel<T, 2>;
+  fold<<<(unsigned)cdiv(n, 64), 64 * kSymvFoldWaves, 0, ctx->stream>>>(n, plan.run, plan.slots, part, alpha,
+                                                                            beta, y, incy);
   WGB_CHECK_LAUNCH("symv_fold_kernel");
   wgb::timing_end(ctx);
   return WGB_OK;
@@ -839,17 +929,16 @@ int trmv(wgb_ctx *ctx, int uplo, int trans, int diag, int64_t n, const T *A, int
   if (incx <= 0 || incy <= 0) return fail(WGB_ERR_INVALID_VALUE, "incx and incy must be positive");
   if (n == 0) return WGB_OK;
   if (!A || !x || !y) return fail(WGB_ERR_INVALID_VALUE, "A, x or y is null");
-  const int64_t nr = cdiv(n, kSymvRows), np = cdiv(n, kSymvPanel);
-  if (np > 65535) return fail(WGB_ERR_INVALID_VALUE, "n too large for one launch");
-  if ((st = wgb::ensure_op_workspace(ctx, (size_t)((np + nr) * n) * sizeof(T)))) return st;
-  T *rowpart = static_cast<T *>(ctx->op_ws);
-  T *colpart = rowpart + np * n;
+  if (n > kSymvMaxN) return fail(WGB_ERR_INVALID_VALUE, "n too large for one launch");
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const SymvPlan plan = uplo == WGB_LOWER ? symv_plan<true>(n, cus) : symv_plan<false>(n, cus);
+  if ((st = wgb::ensure_op_workspace(ctx, (size_t)((plan.slots + cdiv(n, kChunkRows)) * n) * sizeof(T)))) return st;
+  T *part = static_cast<T *>(ctx->op_ws);
   wgb::timing_begin(ctx);
-  const dim3 grid((unsigned)nr, (unsigned)np);
-  const bool vec = lda % 4 == 0 && aligned4(A);
+  const int vec = access_of(n, A, lda);
   const bool lower = uplo == WGB_LOWER, nt = trans == WGB_NO_TRANS, unit = diag == WGB_UNIT;
   auto launch = [&](auto kern) {
-    kern<<<grid, kThreads, 0, ctx->stream>>>(n, A, lda, x, incx, rowpart, colpart);
+    kern<<<(unsigned)plan.blocks, kThreads, 0, ctx->stream>>>(n, plan.run, plan.slots, A, lda, x, incx, part);
   };
   // one instantiation per (vector loads, uplo, form, unit)
   auto pick = [&](auto vec_tag, auto lower_tag, auto mode_tag, auto unit_tag) {
@@ -874,14 +963,16 @@ int trmv(wgb_ctx *ctx, int uplo, int trans, int diag, int64_t n, const T *A, int
     else
       by_mode(v, std::false_type{});
   };
-  if (vec)
-    by_lower(std::true_type{});
+  if (vec == kVecA)
+    by_lower(std::integral_constant<int, kVecA>{});
+  else if (vec == kVecU)
+    by_lower(std::integral_constant<int, kVecU>{});
   else
-    by_lower(std::false_type{});
+    by_lower(std::integral_constant<int, kElems>{});
   WGB_CHECK_LAUNCH("symv_kernel");
   auto fold = [&](auto kern) {
-    kern<<<(unsigned)cdiv(n, kThreads), kThreads, 0, ctx->stream>>>(n, rowpart, colpart, (T)1, (T)0, y,
-                                                                    incy);
+    kern<<<(unsigned)cdiv(n, 64), 64 * kSymvFoldWaves, 0, ctx->stream>>>(n, plan.run, plan.slots, part, (T)1, (T)0, y,
+                                                                         incy);
   };
   if (lower)
     fold(nt ? symv_fold_kernel<T, 1, 1> : symv_fold_kernel<T, 1, 2>);
