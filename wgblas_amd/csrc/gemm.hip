@@ -612,10 +612,15 @@ __device__ __forceinline__ void copies_landed_sync() {
 // loop and the epilogue (unit >= 0: a split-k unit's raw partial to ws).
 // NT = 256 threads (2 x 2 waves); every wave owns a square WT x WT part of
 // the tile.
+//
+// KG > 1: the block is KG groups of NT threads (group kg, smem its own
+// stages), each running the loop over its own k-tiles of the same tile; every
+// group meets the same number of barriers (`idle` more after a loop one
+// k-tile shorter), then the groups' sums are added through LDS in group order.
 template <typename T, int BTM, int BTN, int NT, bool AKC, bool BKC, bool VEC, bool K2 = false,
-          bool SIDE = false>
+          bool SIDE = false, int KG = 1>
 __device__ __forceinline__ void gemm_tile(const GemmArgs<T> &p, int tm, int tn, int unit, int kt0,
-                                          int nkt, T *smem, const int t) {
+                                          int nkt, T *smem, const int t, int kg = 0, bool idle = false) {
   typedef typename Ty<T>::acc Acc;
   typedef typename Ty<T>::v16 V;
   constexpr int VW = Ty<T>::VW;
@@ -1087,6 +1092,30 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs<T> &p, int tm, int tn, 
   else
     mainloop(std::integral_constant<bool, true>{});
 
+  if constexpr (KG > 1) {
+    if (idle) __syncthreads();
+    // every wave is past its last LDS read; group g's sums go to the start
+    // of its own stages (smem), group 0 adds them
+    __syncthreads();
+    static_assert(BTM * BTN <= 2 * STAGE, "a group's sums fit its stages");
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+          *reinterpret_cast<Acc *>(smem + ((i * MB + j) * NT + t) * 4) = acc[i][j];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; ++g)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+          acc[i][j] += *reinterpret_cast<const Acc *>(smem + g * 2 * STAGE + ((i * MB + j) * NT + t) * 4);
+  }
+
   // Epilogue: C = alpha*acc + beta*C on the tile's in-range (and, for
   // sgemmtr/ssyrk, in-triangle) elements.
   if (unit >= 0) {
@@ -1223,6 +1252,26 @@ __global__ __launch_bounds__(kThreads, (VEC || (AKC && BKC) ||
       gemm_tile<T, BT, BT, kThreads, AKC, BKC, VEC, false, true>(p, tm, tn, -1, lo, hi - lo, smem, t);
     }
   }
+}
+
+// fp32 64 x 64 tiles whose k-tiles are shared by KG groups of 4 waves in one
+// block (at least KG k-tiles).
+template <int KG, bool AKC, bool BKC, bool VEC = true>
+__global__ __launch_bounds__(kThreads *KG) void gemm_kgroup_kernel(GemmArgs<float> p) {
+  typedef float T;
+  constexpr int BT = 64, BK = 128 / (int)sizeof(T);
+  constexpr int STAGE = Stager<T, BT, AKC, VEC>::ELEMS + Stager<T, BT, BKC, VEC>::ELEMS;
+  __shared__ __attribute__((aligned(16))) T smem[KG * 2 * STAGE];
+  int tm, tn;
+  logical_tile(xcd_remap(blockIdx.x, p.nregular), p.tiles_m, p.tiles_n, p.uplo, tm, tn);
+  if (tm < 0 || tn < 0 || tm >= p.tiles_m || tn >= p.tiles_n) return;  // block-uniform
+  const int kg = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads);
+  const int nkt_all = (int)((p.k + BK - 1) / BK);
+  const int base = nkt_all / KG, more = nkt_all % KG;  // groups below `more` take one k-tile more
+  const int kt0 = kg * base + (kg < more ? kg : more);
+  gemm_tile<T, BT, BT, kThreads, AKC, BKC, VEC, false, false, KG>(
+      p, tm, tn, -1, kt0, base + (kg < more), smem + kg * 2 * STAGE, (int)threadIdx.x % kThreads, kg,
+      more > 0 && kg >= more);
 }
 
 // Wide fp32 tier: 256 x 128 tiles of C, two blocks of 4 waves per CU, each
@@ -1747,6 +1796,17 @@ KernelFn<T> pick_kernel(bool akc, bool bkc, bool vec, bool pair, bool k2) {
   return pick_layout<T, BT, false>(akc, bkc, vec);
 }
 
+// The k-group kernel of a layout; nullptr where there is none (operands on the
+// register path other than NN).
+template <int KG>
+KernelFn<float> pick_kgroup(bool akc, bool bkc, bool vec) {
+  if (vec) {
+    if (akc) return bkc ? gemm_kgroup_kernel<KG, true, true> : gemm_kgroup_kernel<KG, true, false>;
+    return bkc ? gemm_kgroup_kernel<KG, false, true> : gemm_kgroup_kernel<KG, false, false>;
+  }
+  return !akc && bkc ? gemm_kgroup_kernel<KG, false, true, false> : nullptr;
+}
+
 // Resident blocks per CU of one kernel instantiation (LDS and registers),
 // cached per (tier, operand layout) slot; 0 = not yet queried.
 template <typename T, int BT>
@@ -1811,6 +1871,29 @@ int launch_tier(wgb_ctx *ctx, GemmArgs<T> &a, bool akc, bool bkc, bool vec, WsSo
                                                            (bkc ? 2 : 0) + (vec ? 1 : 0));
   const int64_t nkt = (a.k + BK - 1) / BK;
   a.nregular = a.ntiles;
+  if constexpr (sizeof(T) == 4 && BT == 64) {
+    // Few tiles: one tile per CU leaves one wave per SIMD, whose LDS reads and
+    // copies nothing covers. Two groups of waves share a tile's k-tiles where
+    // every tile has a CU, four over a long k; two also up to two tiles per CU
+    // over a long k, where the second tile already covers most of it. fp32 NT,
+    // one group / two / four: 1024^3 22.2 / 21.1 / 21.1 us, 768^3 17.3 / 16.6 /
+    // 16.7, 640 x 640 x 4096 76.8 / 70.3 / 65.4, 1500 x 1000 x 3000 (384 tiles)
+    // 98.9 / 96.9 / 100.0, but 512 x 4096 x 512 (512 tiles) 20.8 / 21.3 / 24.8.
+    // fp64 keeps one group (two at 1024^3: 36.6 -> 38.2).
+    const bool long_k = nkt >= 64;
+    const int kg = a.ntiles <= cus ? (long_k ? 4 : nkt >= 16 ? 2 : 1) : a.ntiles <= 2 * cus && long_k ? 2 : 1;
+    KernelFn<T> kfn = nullptr;
+    if (kg > 1 && !pair && !k2) kfn = kg == 4 ? pick_kgroup<4>(akc, bkc, vec) : pick_kgroup<2>(akc, bkc, vec);
+    if (kfn) {
+      a.splits = 1;
+      a.kt_split = (int)nkt;
+      a.ws = nullptr;
+      void *args[] = {&a};
+      WGB_CHECK_HIP(hipLaunchKernel(reinterpret_cast<const void *>(kfn), dim3((unsigned)a.ntiles),
+                                    dim3((unsigned)(kg * kThreads)), args, 0, ctx->stream));
+      return WGB_OK;
+    }
+  }
   if (pair) {
     // one block per tile pair (rows r and tiles_m-1-r, or columns), no split
     const bool on_rows = a.band == wgb::kBandALower || a.band == wgb::kBandAUpper;
