@@ -121,7 +121,8 @@ __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t 
                                                               T alpha, T beta,
                                                               T *__restrict__ y, int64_t incy) {
   typedef vec4<T> f4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // (uniform: x entries and column origins stay scalar)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rw = wave % RW, cw = wave / RW;
   const int64_t rb = (int64_t)blockIdx.x * (256 * RW) + 256 * rw + 4 * lane;
   // CW == 1: a lane with fewer than 4 rows reads them one by one instead (the
