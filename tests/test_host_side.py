@@ -1,0 +1,84 @@
+"""The library's host side without a GPU: a stand-in for the HIP runtime
+(tests/native/host_runtime.cc) takes its calls, runs no kernel and keeps a
+list of what was asked of it.
+
+Each check runs in a process of its own, which loads the stand-in ahead of
+libwgblas_hip.so."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, json, sys
+runtime = ctypes.CDLL({runtime!r}, ctypes.RTLD_GLOBAL)
+runtime.standin_log.restype = ctypes.c_char_p
+import wgblas_amd as wg
+from wgblas_amd.native import WgblasError
+
+P = 1 << 41  # a device address
+
+def calls(f):
+    "What f asked of the runtime, line by line, and the error that it raised, if any."
+    runtime.standin_clear()
+    error = None
+    try:
+        f()
+    except WgblasError as e:
+        error = str(e)
+    return runtime.standin_log().decode().splitlines(), error
+
+"""
+
+
+@pytest.fixture(scope="module")
+def child(tmp_path_factory):
+    gxx, hipcc = shutil.which("g++"), shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    include = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc))), "include")
+    if gxx is None or not os.path.exists(os.path.join(include, "hip", "hip_runtime_api.h")):
+        pytest.skip("g++ or the HIP headers are not available")
+    so = str(tmp_path_factory.mktemp("runtime") / "host_runtime.so")
+    subprocess.run([gxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", include,
+                    os.path.join(HERE, "native", "host_runtime.cc"), "-o", so], check=True)
+
+    def run(script):
+        res = subprocess.run([sys.executable, "-c", PRELUDE.format(runtime=so) + script], cwd=ROOT,
+                             capture_output=True, text=True, timeout=300)
+        assert res.returncode == 0, res.stderr
+        return json.loads(res.stdout)
+
+    return run
+
+
+@pytest.mark.parametrize("n", [1, 100_003, 1 << 28])  # one block, one launch, two launches
+def test_a_host_result_that_never_arrives_is_an_error(child, n):
+    """No kernel runs, so nothing stores the result: every host form has to say so instead of
+    returning what the slot holds."""
+    got = child(f"""
+ctx, n, out = wg.Context(0), {n}, {{}}
+for t in "sd":
+    for op in ("dot", "asum", "nrm2", "amax"):
+        name = "i" + t + op if op == "amax" else t + op
+        args = (n, P, 1, P, 1) if op == "dot" else (n, P, 1)
+        out[name] = calls(lambda: getattr(ctx, name)(*args))[1]
+print(json.dumps(out))
+""")
+    assert len(got) == 8
+    for name, error in got.items():
+        assert error and "result" in error and "status -2" in error, (name, error)
+
+
+def test_empty_vectors_need_no_result(child):
+    got = child("""
+ctx = wg.Context(0)
+log, error = calls(lambda: None)
+values = [float(ctx.sdot(0, None, 1, None, 1)), float(ctx.dnrm2(0, None, 1)), ctx.isamax(0, None, 1)]
+print(json.dumps([values, calls(lambda: ctx.sasum(0, None, 1))]))
+""")
+    assert got == [[0.0, 0.0, -1], [[], None]]

@@ -871,10 +871,11 @@ int reduce_to_device(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_
 // Waits for call `seq`'s number in the host slot (four reductions of 100 003
 // floats, host results: copy command and stream wait 76.2 us, stream wait alone
 // 65.4, this 45.9): read directly for as long as a
-// short reduction takes, then (and after an error on the stream, when it never
-// comes) by waiting for the stream, whose own wait costs several us more.
+// short reduction takes, then by waiting for the stream, whose own wait costs
+// several us more. The slot keeps an earlier call's value until this one's
+// arrives, so a stream that ends without it is an error.
 template <class Op>
-int await_result(wgb_ctx *ctx, uint32_t seq, typename Op::Result *result) {
+int await_result(wgb_ctx *ctx, uint32_t seq, typename Op::Result *result, const char *what) {
   typedef std::chrono::steady_clock Clock;
   const uint32_t *word = (const uint32_t *)ctx->host_result + kSeqWord;
   const auto until = Clock::now() + std::chrono::microseconds(kSpinMicros);
@@ -882,7 +883,11 @@ int await_result(wgb_ctx *ctx, uint32_t seq, typename Op::Result *result) {
   do {
     for (int i = 0; i < 64 && !there; ++i) there = __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq;
   } while (!there && Clock::now() < until);
-  if (!there) WGB_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  if (!there) {
+    WGB_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != seq)
+      return wgb::fail(WGB_ERR_HIP, std::string(what) + ": the stream ended without this call's result");
+  }
   *result = *(const typename Op::Result *)ctx->host_result;
   return WGB_OK;
 }
@@ -913,7 +918,7 @@ int reduce_to_host(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t 
   wgb::timing_begin(ctx);
   if ((st = launch_reduce<Op>(ctx, n, x, incx, y, incy, Output<Op>{slot, seq}, what))) return st;
   wgb::timing_end(ctx);
-  return await_result<Op>(ctx, seq, result);
+  return await_result<Op>(ctx, seq, result, what);
 }
 
 }  // namespace
