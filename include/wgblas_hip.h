@@ -388,7 +388,13 @@ int wgb_dgemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, double alpha,
  * positive. The host-result forms block until the value is on the host; the
  * `_dev` forms write the result to device memory and return without
  * synchronising. Both run a fixed two-pass reduction whose summation order
- * depends only on n, so results are reproducible run to run. */
+ * depends only on n, so results are reproducible run to run.
+ *
+ * The reductions of one context share its scratch memory, in the order of its
+ * stream. Under capture the `_dev` forms record kernels only; a graph that
+ * holds some must not be replayed on another stream while the context's own
+ * reductions, or another such graph, may run (either's result may then be
+ * wrong, later calls are not affected), nor after the context is destroyed. */
 
 /* sum x[i*incx]*y[i*incy] in float32. Replaces sdot (src/sdot/sdot.mjs:18-117,
  * src/shaders/sdot.wgsl, src/shaders/reduction/sum.wgsl). */

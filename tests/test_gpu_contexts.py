@@ -7,6 +7,8 @@ of the same handling (the cache keyed by options, which device cleanup(one)
 releases) is checked on the CPU against a host-memory stand-in addon
 (tests/js/devices_cpu.mjs).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -88,3 +90,54 @@ def test_timing_switched_off_and_on(ctx):
         ctx.set_timing(False)
         ctx.synchronize()
         X.free()
+
+
+@pytest.mark.parametrize("n", [4096, 100_003, 1 << 20])
+def test_captured_reductions_replay(n):
+    """The `_dev` reductions under capture (kernels only), replayed on the context's stream with its
+    own eager reductions, and new inputs, between the replays: every replay gives the eager result."""
+    from wgblas_amd import Context
+
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def check(status):
+        assert status == 0, f"HIP status {status}"
+
+    rng = np.random.default_rng(n)
+    with Context(0) as c:
+        stream = ctypes.c_void_p(c.stream)
+        x, y = c.empty(n, np.float32), c.empty(n, np.float32)
+        out, index = c.empty(3, np.float32), c.empty(1, np.int64)
+
+        def reductions():
+            c.sdot_dev(n, x, 1, y, 1, out)
+            c.sasum_dev(n, x, 1, out.offset(1))
+            c.snrm2_dev(n, x, 1, out.offset(2))
+            c.isamax_dev(n, x, 1, index)
+
+        reductions()  # a first launch loads its code object, which a capture must not
+        c.synchronize()
+        graph, executable = ctypes.c_void_p(), ctypes.c_void_p()
+        check(hip.hipStreamBeginCapture(stream, 1))  # thread-local mode
+        try:
+            reductions()
+        finally:
+            check(hip.hipStreamEndCapture(stream, ctypes.byref(graph)))
+        check(hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, ctypes.c_size_t(0)))
+        for replay in range(4):
+            c.h2d(x.ptr, rng.standard_normal(n).astype(np.float32))
+            c.h2d(y.ptr, rng.standard_normal(n).astype(np.float32))
+            reductions()
+            c.synchronize()
+            eager, at = out.to_host(), index.to_host()
+            c.h2d(out.ptr, np.full(3, np.nan, np.float32))
+            host = [c.sdot(n, x, 1, y, 1), c.sasum(n, x, 1), c.snrm2(n, x, 1)]
+            check(hip.hipGraphLaunch(executable, stream))
+            c.synchronize()
+            assert np.array_equal(out.to_host(), eager) and np.array_equal(index.to_host(), at), replay
+            assert np.array_equal(np.array(host, np.float32), eager), replay
+            assert c.isamax(n, x, 1) == at[0]
+        check(hip.hipGraphExecDestroy(executable))
+        check(hip.hipGraphDestroy(graph))
+        for buf in (x, y, out, index):
+            buf.free()

@@ -82,3 +82,34 @@ values = [float(ctx.sdot(0, None, 1, None, 1)), float(ctx.dnrm2(0, None, 1)), ct
 print(json.dumps([values, calls(lambda: ctx.sasum(0, None, 1))]))
 """)
     assert got == [[0.0, 0.0, -1], [[], None]]
+
+
+def test_a_captured_reduction_keeps_no_arrival_count(child):
+    """A captured graph may be replayed on another stream, beside the context's own calls, and a
+    count that two launches share would stay wrong for good: under capture the blocks' partials are
+    folded by a second launch. One block has nothing to count."""
+    got = child("""
+ctx, out = wg.Context(0), []
+for capturing in (0, 1, 0):
+    runtime.standin_capture(capturing)
+    for n, inc in ((4096, 1), (100_003, 1), (100_003, 3), (100_003, 5), (1 << 22, 1)):
+        log, error = calls(lambda: ctx.ddot_dev(n, P, inc, P, inc, P))
+        assert error is None, error
+        out.append([capturing, n, ["fold_kernel" in line for line in log if line.startswith("launch")]])
+print(json.dumps(out))
+""")
+    assert len(got) == 15
+    for capturing, n, launches in got:
+        two = n == 1 << 22 or (capturing and n > 4096)
+        assert launches == ([False, True] if two else [False]), (capturing, n, launches)
+
+
+def test_a_missing_result_clears_the_arrival_count(child):
+    """The next call starts from 0 whatever kept this one from storing its result."""
+    got = child("""
+ctx = wg.Context(0)
+print(json.dumps(calls(lambda: ctx.sasum(100_003, P, 1))[0]))
+""")
+    kinds = [line.split()[0] for line in got]
+    assert kinds == ["launch", "synchronize", "launch"], got
+    assert "set_value" in got[2], got

@@ -505,7 +505,8 @@ __device__ __forceinline__ P load_partial(const P *slot) {
 // The arrival is ordered after the partial by waiting for the stores
 // (s_waitcnt vmcnt(0)): a release fence at agent scope would write back the
 // XCD's L2 in every block (~90 us per 2048-block launch on MI355X).
-// The last block sets the counter back to 0 for the stream's next launch.
+// The last block sets the counter back to 0 for the stream's next launch
+// (captured launches of several blocks never count: fused_limit).
 template <class Op>
 __device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Partial *partials,
                                        uint32_t *arrived, Output<Op> out) {
@@ -806,6 +807,18 @@ void *arrival_counter(wgb_ctx *ctx) {
   return (char *)ctx->scratch + (size_t)wgb::kMaxReduceBlocks * kPartialBytes;
 }
 
+// The most first-pass blocks whose partials this call may fold in the same
+// launch. The context's stream orders the launches that count arrivals, but a
+// captured graph may be replayed on another stream, beside them: a count that
+// two launches share would stay off zero for every later call. Captured
+// launches therefore keep none (one block has nothing to count).
+int fused_limit(wgb_ctx *ctx, int *blocks) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  WGB_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &status));
+  *blocks = status == hipStreamCaptureStatusNone ? kMaxFusedBlocks : 1;
+  return WGB_OK;
+}
+
 // Stage 1 (the read pass) and stage 2 (the fold): one launch for few blocks,
 // else two on the stream.
 template <class Op>
@@ -814,19 +827,21 @@ int launch_reduce(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t i
                   const char *what) {
   static_assert(sizeof(typename Op::Partial) <= kPartialBytes, "partial slot too small");
   const int G = reduce_blocks(n);
+  int most = 0, st;
+  if ((st = fused_limit(ctx, &most))) return st;
   auto *part = (typename Op::Partial *)partials_of(ctx);
   int Gl = G;
   const bool same = Op::NIN == 1 || (incy == incx && aligned16(y));
   const int64_t span = (n - 1) * incx + 1;
   auto *arrived = (uint32_t *)arrival_counter(ctx);
   const Output<Op> unfused = {nullptr, 0};
-  Output<Op> fused = G <= kMaxFusedBlocks ? out : unfused;
+  Output<Op> fused = G <= most ? out : unfused;
   if (incx == 1 && aligned16(x) && same) {
     reduce_vec<Op><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
   } else if (incx >= 2 && incx <= 4 && aligned16(x) && same && span < ((int64_t)1 << 31)) {
     // G from the span, not n: each block reads a span range.
     Gl = reduce_blocks(span);
-    fused = Gl <= kMaxFusedBlocks ? out : unfused;
+    fused = Gl <= most ? out : unfused;
     if (incx == 2)
       reduce_span<Op, 2><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
     else if (incx == 3)
@@ -873,7 +888,8 @@ int reduce_to_device(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_
 // 65.4, this 45.9): read directly for as long as a
 // short reduction takes, then by waiting for the stream, whose own wait costs
 // several us more. The slot keeps an earlier call's value until this one's
-// arrives, so a stream that ends without it is an error.
+// arrives, so a stream that ends without it is an error; the count of arrivals
+// is then cleared for the next call.
 template <class Op>
 int await_result(wgb_ctx *ctx, uint32_t seq, typename Op::Result *result, const char *what) {
   typedef std::chrono::steady_clock Clock;
@@ -885,8 +901,10 @@ int await_result(wgb_ctx *ctx, uint32_t seq, typename Op::Result *result, const 
   } while (!there && Clock::now() < until);
   if (!there) {
     WGB_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != seq)
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != seq) {
+      set_value<<<1, 1, 0, ctx->stream>>>((uint32_t *)arrival_counter(ctx), 0u);
       return wgb::fail(WGB_ERR_HIP, std::string(what) + ": the stream ended without this call's result");
+    }
   }
   *result = *(const typename Op::Result *)ctx->host_result;
   return WGB_OK;
