@@ -113,3 +113,12 @@ print(json.dumps(calls(lambda: ctx.sasum(100_003, P, 1))[0]))
     kinds = [line.split()[0] for line in got]
     assert kinds == ["launch", "synchronize", "launch"], got
     assert "set_value" in got[2], got
+
+
+def test_the_result_slot_is_coherent_memory(child):
+    """A kernel's stores to the slot are read while its stream goes on, which only coherent host
+    memory allows; without the flag the runtime's environment may choose otherwise."""
+    got = child("print(json.dumps(calls(lambda: wg.Context(0))[0]))")
+    flags = [int(line.split()[2]) for line in got if line.startswith("host_malloc")]
+    coherent, non_coherent = 0x40000000, 0x80000000
+    assert len(flags) == 1 and flags[0] & coherent and not flags[0] & non_coherent, got

@@ -122,7 +122,8 @@ extern "C" int wgb_init(int device, wgb_ctx **out) {
   // the reductions' arrival counter starts at 0
   if (e == hipSuccess) e = hipMemsetAsync(ctx->scratch, 0, wgb::kScratchBytes, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  if (e == hipSuccess) e = hipHostMalloc(&ctx->host_result, 64, hipHostMallocDefault);
+  // coherent: kernels' stores are read while the stream goes on
+  if (e == hipSuccess) e = hipHostMalloc(&ctx->host_result, 64, hipHostMallocCoherent);
   if (e == hipSuccess) std::memset(ctx->host_result, 0, 64);
   if (e != hipSuccess) {
     int st = wgb::fail_hip(e, "wgb_init");
