@@ -122,3 +122,23 @@ def test_the_result_slot_is_coherent_memory(child):
     flags = [int(line.split()[2]) for line in got if line.startswith("host_malloc")]
     coherent, non_coherent = 0x40000000, 0x80000000
     assert len(flags) == 1 and flags[0] & coherent and not flags[0] & non_coherent, got
+
+
+def test_reductions_fold_in_the_same_launch_only_where_that_is_no_slower(child):
+    """Sums of one word up to 256 first-pass blocks of 4096 elements, folds of more words and
+    strided reads up to 192, strided reads of 8-byte elements up to 128."""
+    got = child("""
+ctx, out = wg.Context(0), []
+for name, two, blocks, inc in (("sdot", 1, 256, 1), ("ddot", 1, 256, 1), ("dasum", 0, 256, 1), ("snrm2", 0, 192, 1),
+                               ("dnrm2", 0, 192, 1), ("isamax", 0, 192, 1), ("idamax", 0, 192, 1),
+                               ("ddot", 1, 128, 5), ("sasum", 0, 192, 7), ("dnrm2", 0, 128, 6)):
+    for n in (blocks * 4096, blocks * 4096 + 1):
+        args = (n, P, inc, P, inc, P) if two else (n, P, inc, P)
+        log, error = calls(lambda: getattr(ctx, name + "_dev")(*args))
+        assert error is None, error
+        out.append([name, inc, n > blocks * 4096, sum(line.startswith("launch") for line in log)])
+print(json.dumps(out))
+""")
+    assert len(got) == 20
+    for name, inc, above, launches in got:
+        assert launches == (2 if above else 1), (name, inc, above, launches)

@@ -67,11 +67,17 @@ constexpr int kUnroll = 16;
 constexpr int kTail = 4;  // loads in flight over what is left of a range
 constexpr int64_t kElemsPerBlockMin = 4096;
 // Up to this many first-pass blocks the last one to arrive folds (one launch).
-// The arrivals serialise on one word, about 10 ns each, against about 2 us
-// for the second launch: four reductions of fp32 vectors, both ways, 245 blocks
-// (n = 10^6) 26.3 us fused and 29.9 in two launches, 977 blocks (4 10^6) 62.8
-// and 29.1, 4096 blocks (2^28) 911 and 770.
+// The arrivals serialise on one word, about 10 ns each, and the fold comes
+// after them, against a second launch that costs about 2 us where launches are
+// what a call waits for and little where the read hides it. One launch / two,
+// us a call, results left in device memory, on two boxes whose launches differ:
+// sdot 256 blocks 6.4 / 6.6, dasum 256 7.1 / 7.7; folds of more than one word
+// cost more: isamax 192 blocks 6.4 / 6.3 and 6.4 / 7.3, 224 6.8 / 6.3 and 6.8 /
+// 7.3, dnrm2 192 7.8 / 7.8, 224 8.2 / 7.8; strided reads are longer: sdot, stride
+// 5, 192 blocks 6.8 / 7.2, 245 9.9 / 9.2, ddot 128 9.6 / 9.7, 160 11.4 / 11.0.
 constexpr int kMaxFusedBlocks = 256;
+constexpr int kMaxFusedDear = 192;      // more than one word to fold, or a strided read
+constexpr int kMaxFusedStrided8 = 128;  // a strided read of 8-byte elements
 
 // snrm2 thresholds and scales (powers of two): src/shaders/snrm2.wgsl:33-36.
 constexpr float kTsml = 0x1p-63f;
@@ -506,7 +512,7 @@ __device__ __forceinline__ P load_partial(const P *slot) {
 // (s_waitcnt vmcnt(0)): a release fence at agent scope would write back the
 // XCD's L2 in every block (~90 us per 2048-block launch on MI355X).
 // The last block sets the counter back to 0 for the stream's next launch
-// (captured launches of several blocks never count: fused_limit).
+// (captured launches of several blocks never count: fuse_fold).
 template <class Op>
 __device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Partial *partials,
                                        uint32_t *arrived, Output<Op> out) {
@@ -807,15 +813,17 @@ void *arrival_counter(wgb_ctx *ctx) {
   return (char *)ctx->scratch + (size_t)wgb::kMaxReduceBlocks * kPartialBytes;
 }
 
-// The most first-pass blocks whose partials this call may fold in the same
+// Whether a call of G first-pass blocks, at most `most`, folds in the same
 // launch. The context's stream orders the launches that count arrivals, but a
 // captured graph may be replayed on another stream, beside them: a count that
 // two launches share would stay off zero for every later call. Captured
 // launches therefore keep none (one block has nothing to count).
-int fused_limit(wgb_ctx *ctx, int *blocks) {
+int fuse_fold(wgb_ctx *ctx, int G, int most, bool *fuse) {
+  *fuse = G <= most;
+  if (!*fuse || G == 1) return WGB_OK;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   WGB_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &status));
-  *blocks = status == hipStreamCaptureStatusNone ? kMaxFusedBlocks : 1;
+  *fuse = status == hipStreamCaptureStatusNone;
   return WGB_OK;
 }
 
@@ -826,34 +834,34 @@ int launch_reduce(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t i
                   const typename Op::Elem *y, int64_t incy, Output<Op> out,
                   const char *what) {
   static_assert(sizeof(typename Op::Partial) <= kPartialBytes, "partial slot too small");
-  const int G = reduce_blocks(n);
-  int most = 0, st;
-  if ((st = fused_limit(ctx, &most))) return st;
   auto *part = (typename Op::Partial *)partials_of(ctx);
-  int Gl = G;
+  auto *arrived = (uint32_t *)arrival_counter(ctx);
   const bool same = Op::NIN == 1 || (incy == incx && aligned16(y));
   const int64_t span = (n - 1) * incx + 1;
-  auto *arrived = (uint32_t *)arrival_counter(ctx);
-  const Output<Op> unfused = {nullptr, 0};
-  Output<Op> fused = G <= most ? out : unfused;
-  if (incx == 1 && aligned16(x) && same) {
+  const bool vec = incx == 1 && aligned16(x) && same;
+  const bool by_span = incx >= 2 && incx <= 4 && aligned16(x) && same && span < ((int64_t)1 << 31);
+  // G from the span, not n, where each block reads a span range.
+  const int G = reduce_blocks(by_span ? span : n);
+  const bool strided = !vec && !by_span && (incx > 1 || (Op::NIN == 2 && incy > 1));
+  const int most = strided && sizeof(typename Op::Elem) == 8 ? kMaxFusedStrided8
+                   : strided || sizeof(typename Op::Partial) > 8 ? kMaxFusedDear : kMaxFusedBlocks;
+  bool fuse = false;
+  int st;
+  if ((st = fuse_fold(ctx, G, most, &fuse))) return st;
+  const Output<Op> fused = fuse ? out : Output<Op>{nullptr, 0};
+  if (vec)
     reduce_vec<Op><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
-  } else if (incx >= 2 && incx <= 4 && aligned16(x) && same && span < ((int64_t)1 << 31)) {
-    // G from the span, not n: each block reads a span range.
-    Gl = reduce_blocks(span);
-    fused = Gl <= most ? out : unfused;
-    if (incx == 2)
-      reduce_span<Op, 2><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
-    else if (incx == 3)
-      reduce_span<Op, 3><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
-    else
-      reduce_span<Op, 4><<<Gl, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
-  } else {
+  else if (by_span && incx == 2)
+    reduce_span<Op, 2><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
+  else if (by_span && incx == 3)
+    reduce_span<Op, 3><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
+  else if (by_span)
+    reduce_span<Op, 4><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
+  else
     reduce_strided<Op><<<G, kThreads, 0, ctx->stream>>>(x, incx, y, incy, n, part, arrived, fused);
-  }
   WGB_CHECK_LAUNCH(what);
-  if (fused.ptr) return WGB_OK;
-  fold_kernel<Op><<<1, kThreads, 0, ctx->stream>>>(part, Gl, out);
+  if (fuse) return WGB_OK;
+  fold_kernel<Op><<<1, kThreads, 0, ctx->stream>>>(part, G, out);
   WGB_CHECK_LAUNCH(what);
   return WGB_OK;
 }
