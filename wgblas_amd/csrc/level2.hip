@@ -771,12 +771,18 @@ __global__ __launch_bounds__(kThreads) void symv_kernel(int64_t n, int64_t run, 
   };
   auto range = [&](auto cross_tag, int64_t ja, int64_t jb) {
     if (ja >= jb) return;
+    // symv: only a run's last, partial step has run-time columns. A wave that
+    // crosses n and took them for its 256 diagonal columns set the launch's time
+    // (ssymv 16383 upper, lda 16384, 151 us against 89 now; lower 12000 90
+    // against 51). strmv keeps them there: its shorter kernels lose 2 to 4% to
+    // the form's code at orders that are multiples of 256.
+    constexpr bool CROSS = decltype(cross_tag)::value;
     const bool all = w0 + 256 <= n;
-    const int64_t jw = VEC && (all || !decltype(cross_tag)::value) ? ja + (jb - ja) / S * S : ja;
+    const int64_t jw = VEC && (all || !CROSS || MODE == 0) ? ja + (jb - ja) / S * S : ja;
     if (ja < jw) {
       if (all)
         steps(std::true_type{}, cross_tag, std::false_type{}, ja, jw);
-      else if constexpr (!decltype(cross_tag)::value)
+      else if constexpr (!CROSS || MODE == 0)
         steps(std::true_type{}, cross_tag, std::true_type{}, ja, jw);
     }
     if (jw < jb) steps(std::false_type{}, std::true_type{}, std::false_type{}, jw, jb);
