@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
   const int64_t ib = r0 + 4 * threadIdx.x;  // the lane's own rows start here
   if (ib >= m) return;
   // VEC not kElems (m >= 4): a lane whose rows cross m takes the matrix's last 4 rows, in
-  // bounds, and stores only its own, [lo, 4) of them
+  // bounds; [lo, 4) of them are its own
   const int64_t i0 = VEC && ib > m - 4 ? m - 4 : ib;
   const int lo = (int)(ib - i0);
   const int rows = i0 + 4 <= m ? 4 : (int)(m - i0);
@@ -407,17 +407,20 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
       if (TWO) a[q] = fma(yv[q], t2, a[q]);
     }
   };
-  // FULL: every row of the wave inside m (a wave-uniform choice): whole
-  // non-temporal vectors with no per-lane branch between the stores. The loads
-  // are whole vectors in either case (m >= 4), at any alignment of A and lda.
-  // MASK (the diagonal columns of a triangle): the same loads and arithmetic,
-  // and each lane stores only its rows inside the triangle (whole vectors
-  // where all four are).
-  auto walk = [&](auto full_tag, auto mask_tag, int64_t ja, int64_t jb) {
-    constexpr bool FULL = decltype(full_tag)::value;
+  // MODE: how the wave accesses A, whole vectors with no per-lane branch
+  // between the stores (kVecA: non-temporal), or kElems for a wave with fewer
+  // than 4 rows (its loads are still whole vectors where m >= 4) or a matrix with
+  // fewer. A lane whose rows cross m updates the last 4 rows of its wave, as its
+  // neighbours in the same instructions do: the rows they share get the same
+  // values. MASK (the diagonal columns of a triangle): the same loads and
+  // arithmetic, and each lane stores only its own rows inside the triangle (whole
+  // vectors where all four are).
+  auto walk = [&](auto mode_tag, auto mask_tag, int64_t ja, int64_t jb) {
+    constexpr int MODE = decltype(mode_tag)::value;
+    constexpr bool FULL = MODE != kElems;
     constexpr bool MASK = decltype(mask_tag)::value;
     auto load = [&](const T *col) -> f4 {
-      if constexpr (VEC) return ld<FULL ? VEC : kVecU>(col + i0);
+      if constexpr (VEC) return ld<FULL ? MODE : kVecU>(col + i0);
       f4 v;
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = col[i0 + (q < rows ? q : 0)];
@@ -436,7 +439,7 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
         }
       }
       if (FULL || (VEC && lo == 0)) {
-        if constexpr (FULL && VEC == kVecA)
+        if constexpr (MODE == kVecA)
           __builtin_nontemporal_store(v, reinterpret_cast<vec4u<T> *>(col + i0));
         else
           *reinterpret_cast<vec4u<T> *>(col + i0) = v;
@@ -472,15 +475,22 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
       }
     }
   };
-  // a wave's choice: the one wave that crosses m is the only slow one
   const int64_t w0 = r0 + 256 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the wave's 256 rows
-  const bool whole_rows = VEC && w0 + 256 <= m;
+  const bool vectors = VEC && m - w0 >= 4;
+  // The blocks of a row chunk that m cuts access A through the caches: non-temporal
+  // whole waves there and element stores in the crossing one took dger 768 x
+  // 30000 87 us (element accesses in the whole block 71, this 58), 1001 x 30000,
+  // lda 1004, 103 (93, 74), 5001^2, lda 5004, 112 (108, 107), 8191^2, lda 8192, 198
+  // (192, 192).
+  const bool cut = r0 + kChunkRows > m;
   auto walk_range = [&](auto mask_tag, int64_t ja, int64_t jb) {
     if (ja >= jb) return;
-    if (whole_rows)
-      walk(std::true_type{}, mask_tag, ja, jb);
+    if (vectors && !cut)
+      walk(std::integral_constant<int, VEC>{}, mask_tag, ja, jb);
+    else if (vectors)
+      walk(std::integral_constant<int, VEC ? kVecU : kElems>{}, mask_tag, ja, jb);
     else
-      walk(std::false_type{}, mask_tag, ja, jb);
+      walk(std::integral_constant<int, kElems>{}, mask_tag, ja, jb);
   };
   // columns wholly inside the triangle for these 256 rows, and diagonal ones
   // (row i of column j is stored where i >= j (lower) or i <= j (upper))
