@@ -142,3 +142,21 @@ print(json.dumps(out))
     assert len(got) == 20
     for name, inc, above, launches in got:
         assert launches == (2 if above else 1), (name, inc, above, launches)
+
+
+def test_transposed_gemv_accesses_by_alignment(child):
+    """Aligned columns: vectors past the caches (2). Others: element by element (0) below 64 rows, else vectors
+    through the caches (1), or past them in fp32 where A is larger than they are. A strided x: by element."""
+    got = child("""
+ctx, out = wg.Context(0), []
+for name in ("sgemv", "dgemv"):
+    for m, n, lda, shift, incx in ((300, 300, 300, 0, 1), (300, 300, 300, 8, 1), (300, 300, 301, 0, 1), (5000, 5000, 5002, 0, 1),
+                                   (300, 300, 300, 0, 2), (60, 9000, 60, 0, 1), (63, 9000, 65, 0, 1), (64, 9000, 65, 0, 1),
+                                   (8191, 8191, 8191, 0, 1), (8191, 8194, 8193, 0, 1)):
+        log, error = calls(lambda: getattr(ctx, name)(1, m, n, 1.0, P + shift, lda, P, incx, 0.0, P, 1))
+        assert error is None, error
+        out.append(next(line.split()[-1] for line in log if "gemv_t_kernel" in line))
+print(json.dumps(out))
+""")
+    kinds = [name.split("gemv_t_kernelI")[1][:4] for name in got]
+    assert kinds == ["fLi" + k for k in "2111020112"] + ["dLi" + k for k in "2111020111"], kinds

@@ -93,9 +93,29 @@ __device__ __forceinline__ vec4<T> ld(const T *p) {
 }
 
 template <typename T>
-int access_of(int64_t rows, const T *A, int64_t lda) {
-  if (rows < 4) return kElems;
+int vector_access(const T *A, int64_t lda) {
   return lda % 4 == 0 && (uintptr_t)A % (4 * sizeof(T)) == 0 ? kVecA : kVecU;
+}
+
+template <typename T>
+int access_of(int64_t rows, const T *A, int64_t lda) {
+  return rows < 4 ? kElems : vector_access(A, lda);
+}
+
+// gemv T's access (incx == 1). Unaligned columns: element by element below 64 rows
+// (a column is then a few lines, most of them shared with its neighbours:
+// sgemv 33 x 1000001, lda 37, elements 92 us, vectors 99, non-temporal ones
+// 122), else vectors; through the caches where they can hold A or in fp64, whose
+// vectors are two lines wide (non-temporal / not: sgemv 2048^2, lda 2049, 9.0 /
+// 8.5, 8191^2 49 / 45, 2001 x 60001 74 / 79, 12001^2 97 / 102; dgemv 2048^2 14.0 /
+// 10.7, elements 13.1, 4096^2 31 / 28, 8191^2 103 / 101).
+constexpr int64_t kCacheBytes = (int64_t)256 << 20;
+template <typename T>
+int access_t(int64_t m, int64_t n, const T *A, int64_t lda) {
+  const int vec = vector_access(A, lda);
+  if (vec == kVecA) return kVecA;
+  if (m < 64) return kElems;
+  return sizeof(T) == 8 || lda * n <= kCacheBytes / (int64_t)sizeof(T) ? kVecU : kVecA;
 }
 
 // Writes one output element: alpha * acc + beta * y (beta == 0 never reads y).
@@ -192,8 +212,10 @@ __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t 
 }
 
 // T form. Wave w (4 per block) owns columns [CPW w, CPW w + CPW) of split s, rows
-// [s*rps, min(m, (s+1)*rps)). VEC: incx == 1 (A, lda and x at any alignment).
-template <typename T, bool VEC, int CPW>
+// [s*rps, min(m, (s+1)*rps)). VEC not kElems: incx == 1, vectors of A and x at any
+// alignment (rows past a split's last whole vector one by one); access_t says
+// which.
+template <typename T, int VEC, int CPW>
 __global__ __launch_bounds__(kThreads) void gemv_t_kernel(int64_t m, int64_t n,
                                                           const T *__restrict__ A, int64_t lda,
                                                           const T *__restrict__ x, int64_t incx,
@@ -222,8 +244,8 @@ __global__ __launch_bounds__(kThreads) void gemv_t_kernel(int64_t m, int64_t n,
       f4 av0[CPW], av1[CPW];
 #pragma unroll
       for (int c = 0; c < CPW; ++c) {
-        av0[c] = ld_nt(col[c] + i);
-        av1[c] = ld_nt(col[c] + i + 256);
+        av0[c] = ld<VEC>(col[c] + i);
+        av1[c] = ld<VEC>(col[c] + i + 256);
       }
       // fp64: every load of the step is issued before the arithmetic. Left
       // to itself the scheduler placed each 16-byte load just before its
@@ -244,7 +266,7 @@ __global__ __launch_bounds__(kThreads) void gemv_t_kernel(int64_t m, int64_t n,
       const f4 xv = *reinterpret_cast<const vec4u<T> *>(x + i);
       f4 av[CPW];
 #pragma unroll
-      for (int c = 0; c < CPW; ++c) av[c] = ld_nt(col[c] + i);
+      for (int c = 0; c < CPW; ++c) av[c] = ld<VEC>(col[c] + i);
 #pragma unroll
       for (int c = 0; c < CPW; ++c)
 #pragma unroll
@@ -1079,14 +1101,18 @@ int gemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, T alpha, const T *A, int
              kThreads);
     WGB_CHECK_LAUNCH("gemv_n_kernel");
   } else {
-    const bool vec = incx == 1;
-    auto launch = [&](auto kern) {
+    const int vec = incx != 1 ? kElems : access_t(m, n, A, lda);
+    auto launch = [&](auto vec_tag) {
+      constexpr int VEC = decltype(vec_tag)::value;
+      auto kern = cpw == kColsPerWaveShort ? gemv_t_kernel<T, VEC, kColsPerWaveShort> : gemv_t_kernel<T, VEC, kColsPerWave>;
       kern<<<grid, kThreads, 0, ctx->stream>>>(m, n, A, lda, x, incx, per, part, alpha, beta, y, incy);
     };
-    if (cpw == kColsPerWaveShort)
-      launch(vec ? gemv_t_kernel<T, true, kColsPerWaveShort> : gemv_t_kernel<T, false, kColsPerWaveShort>);
+    if (vec == kVecA)
+      launch(std::integral_constant<int, kVecA>{});
+    else if (vec == kVecU)
+      launch(std::integral_constant<int, kVecU>{});
     else
-      launch(vec ? gemv_t_kernel<T, true, kColsPerWave> : gemv_t_kernel<T, false, kColsPerWave>);
+      launch(std::integral_constant<int, kElems>{});
     WGB_CHECK_LAUNCH("gemv_t_kernel");
   }
   if (part) {
