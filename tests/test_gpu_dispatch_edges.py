@@ -96,6 +96,26 @@ def test_level2_edges(ctx, prefix, dtype, n, pad):
     assert np.array_equal(dG.to_host().reshape(n, lda), want)
 
 
+@pytest.mark.parametrize("prefix,dtype", [("s", np.float32), ("d", np.float64)])
+@pytest.mark.parametrize("m,n,lda", [(1024, 65536, 1024), (1027, 33001, 1027), (1027, 33001, 1028), (2050, 32770, 2052),
+                                     (1279, 32765, 1280), (3, 66001, 3), (4097, 13003, 4097)])
+def test_gemv_wide_blocks(ctx, prefix, dtype, m, n, lda):
+    """1024-row blocks over many columns: whole waves, waves that cross m (by rows m % 4 and by whole lanes), fewer
+    rows than a vector, columns that are no multiple of the step, each alignment."""
+    rng = np.random.default_rng(m + n + lda)
+    A = _ints(rng, (n, lda), np.int8)  # row j is column j; whole numbers, |sums| <= 49 n + 7 < 2^24
+    x, y = _ints(rng, n, dtype), _ints(rng, m, dtype)
+    x[rng.random(n) < 0.2] = 0
+    dA, dx, dy = ctx.upload(A.astype(dtype)), ctx.upload(x), ctx.upload(y)
+    try:
+        getattr(ctx, prefix + "gemv")(0, m, n, 2.0, dA, lda, dx, 1, -1.0, dy, 1)
+        want = 2.0 * (x.astype(np.float64) @ A[:, :m].astype(np.float64)) - y
+        assert np.array_equal(dy.to_host(), want)
+    finally:
+        for buf in (dA, dx, dy):
+            buf.free()
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("m,n,k", [(1024, 1024, 256), (1000, 1025, 263), (1024, 1024, 545), (900, 1100, 1090),
                                    (1500, 1400, 301), (2048, 1024, 320)])

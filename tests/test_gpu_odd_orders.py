@@ -62,3 +62,19 @@ def test_dger_with_a_cut_row_chunk(timed, rows, lda, limit):
     finally:
         for buf in (A, x, y):
             buf.free()
+
+
+# 1.94 with the fault, 1.0 without
+@pytest.mark.parametrize("m,lda", [(8191, 8191), (8189, 8190)])
+def test_dgemv_at_rows_that_are_no_multiple_of_4(timed, m, lda):
+    c = timed
+    A, x, y = c.empty(8192 * 8192, np.float64), c.empty(8192, np.float64), c.empty(8192, np.float64)
+    try:
+        for k, buf in enumerate((A, x, y)):
+            c.fill_uniform(buf, -1, 1, 27 + k)
+        odd = _best(c, lambda: c.dgemv(0, m, 8191, 1.0, A, lda, x, 1, 0.0, y, 1))
+        even = _best(c, lambda: c.dgemv(0, 8192, 8192, 1.0, A, 8192, x, 1, 0.0, y, 1))
+        assert odd < LIMIT * even, (odd, even)
+    finally:
+        for buf in (A, x, y):
+            buf.free()

@@ -102,6 +102,27 @@ int access_of(int64_t rows, const T *A, int64_t lda) {
   return rows < 4 ? kElems : vector_access(A, lda);
 }
 
+// Pins a value in its register(s) here: nothing before this point is moved past
+// it. held_scalar: a value that is the same in every lane, in scalar registers.
+template <typename T>
+__device__ __forceinline__ T held(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ T held_scalar(T v) {
+  constexpr int W = sizeof(T) / 4;
+  int w[W];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    w[k] = __builtin_amdgcn_readfirstlane(w[k]);
+    asm volatile("" : "+s"(w[k]));
+  }
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+
 // gemv T's access (incx == 1). Unaligned columns: element by element below 64 rows
 // (a column is then a few lines, most of them shared with its neighbours:
 // sgemv 33 x 1000001, lda 37, elements 92 us, vectors 99, non-temporal ones
@@ -133,6 +154,16 @@ __device__ __forceinline__ void store_y(T *y, int64_t idx, T acc, T alpha, T bet
 // multiple of CW kStepN where CW > 1; the CW partial sums of a row are added through LDS in wave
 // order. VEC not kElems (m >= 4): a lane whose rows cross m (or lie past it) reads
 // the matrix's last 4 rows instead, in bounds, and stores only its own.
+//
+// The wide blocks' (CW == 1) whole waves keep every load of a step in flight
+// before its arithmetic, in the form that measured best for the type: in fp32
+// behind a per-lane branch that every lane of theirs takes, in fp64 by reading
+// the x entries and then the columns into registers before the first is used.
+// (fp32 20480^2 297 us, with fp64's form 332; fp64 16384^2 336, with fp32's 560.)
+// Left to itself the compiler sinks each load of A and x into the branch on its
+// column's x entry (fp64 512 x 200000 192 us). The wave that crosses m has its own loop: as
+// a per-lane choice between vectors and elements it ran both for each column,
+// and the launch waited for it (dgemv 8191^2, lda 8191, 183 us; now 93).
 template <typename T, int VEC, int RW, int CW>
 __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t n,
                                                               const T *__restrict__ A, int64_t lda,
@@ -141,25 +172,25 @@ __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t 
                                                               T alpha, T beta,
                                                               T *__restrict__ y, int64_t incy) {
   typedef vec4<T> f4;
+  constexpr bool HELD = CW == 1 && sizeof(T) == 8;    // a step's operands held before its arithmetic
+  constexpr bool BRANCH = CW == 1 && sizeof(T) == 4;  // whole waves load behind a per-lane branch
   // (uniform: x entries and column origins stay scalar)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rw = wave % RW, cw = wave / RW;
-  const int64_t rb = (int64_t)blockIdx.x * (256 * RW) + 256 * rw + 4 * lane;
-  // CW == 1: a lane with fewer than 4 rows reads them one by one instead (the
-  // per-lane branch keeps each step's loads together: 16384^2 161 us fp32, 333
-  // fp64, against 171 and 342 with the clamped vectors)
-  const bool whole = rb + 4 <= m;
-  if (CW == 1 && rb >= m) return;
-  const int64_t i0 = VEC && CW > 1 ? (rb <= m - 4 ? rb : m - 4) : (rb < m ? rb : 0);
+  const int64_t wr = (int64_t)blockIdx.x * (256 * RW) + 256 * rw;  // the wave's rows start here
+  const int64_t rb = wr + 4 * lane;
+  if (CW == 1 && wr >= m) return;
+  const int64_t i0 = VEC ? (rb <= m - 4 ? rb : m - 4) : (rb < m ? rb : 0);
   int64_t j = (int64_t)blockIdx.y * cps;
   int64_t j1 = j + cps < n ? j + cps : n;
   j += cw * (cps / CW);
   if (CW > 1 && j1 > j + cps / CW) j1 = j + cps / CW;
   T acc[4] = {(T)0, (T)0, (T)0, (T)0};
-  // kStepN columns per step, every load issued before the arithmetic. LAST:
-  // columns past j1 repeat the last one against a zero x entry, which skips them
-  auto step = [&](auto last_tag) {
-    constexpr bool LAST = decltype(last_tag)::value;
+  // kStepN columns per step. LAST: columns past j1 repeat the last one against a
+  // zero x entry, which skips them
+  auto step = [&](auto last_tag, auto whole_tag) {
+    constexpr bool LAST = decltype(last_tag)::value, WHOLE = decltype(whole_tag)::value;
+    const int64_t i = WHOLE && HELD ? rb : i0;
     T xv[kStepN];
     f4 av[kStepN];
 #pragma unroll
@@ -170,12 +201,20 @@ __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t 
 #pragma unroll
     for (int c = 0; c < kStepN; ++c) {
       const T *col = A + (!LAST || j + c < j1 ? j + c : j1 - 1) * lda;
-      if (VEC && (CW > 1 || whole)) {
-        av[c] = ld<VEC>(col + i0);
+      if (WHOLE && BRANCH ? rb + 4 <= m : VEC != kElems) {
+        av[c] = ld<VEC>(col + i);
       } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) av[c][q] = col[i0 + q < m ? i0 + q : m - 1];
+        for (int q = 0; q < 4; ++q) av[c][q] = col[i + q < m ? i + q : m - 1];
       }
+    }
+    if constexpr (HELD) {
+#pragma unroll
+      for (int c = 0; c < kStepN; ++c) xv[c] = held_scalar(xv[c]);
+#pragma unroll
+      for (int c = 0; c < kStepN; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) av[c][q] = held(av[c][q]);
     }
 #pragma unroll
     for (int c = 0; c < kStepN; ++c) {
@@ -185,8 +224,14 @@ __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t 
       }
     }
   };
-  for (; j + kStepN <= j1; j += kStepN) step(std::false_type{});
-  if (j < j1) step(std::true_type{});
+  auto walk = [&](auto whole_tag) {
+    for (; j + kStepN <= j1; j += kStepN) step(std::false_type{}, whole_tag);
+    if (j < j1) step(std::true_type{}, whole_tag);
+  };
+  if (CW == 1 && VEC && wr + 256 <= m)  // a wave's choice
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
   if constexpr (CW > 1) {
     __shared__ T red[CW - 1][RW * 64][4];
     if (cw > 0) {
