@@ -160,3 +160,41 @@ print(json.dumps(out))
 """)
     kinds = [name.split("gemv_t_kernelI")[1][:4] for name in got]
     assert kinds == ["fLi" + k for k in "2111020112"] + ["dLi" + k for k in "2111020111"], kinds
+
+
+def test_gemv_blocks_by_the_busiest_cu(child):
+    """gemv N's two kinds of block, 256 rows (1 x 8 waves) or 1024 (4 x 1), on both sides of each
+    of the rule's lines; with one block per CU or fewer beside each other, no CU gets two."""
+    shapes = {
+        # narrow in both
+        (4096, 4096): "nn", (2000, 30000): "nn", (7000, 7000): "nn", (50000, 768): "nn", (300, 1000): "nn",
+        # few rows, whatever the columns
+        (1, 200000): "nn", (250, 70000): "nn", (512, 160000): "nn", (513, 160000): "ww",
+        # the wide blocks fill the CUs
+        (8192, 8192): "ww", (16384, 16384): "ww", (1025, 40000): "ww", (400000, 10): "ww",
+        # splits that do not divide the CUs' work evenly
+        (15000, 4000): "ww", (25000, 2304): "ww", (1024, 57000): "nn", (1024, 65000): "nw",
+        (964, 61000): "nw", (800, 65000): "nw",
+        # more than one narrow block per CU beside each other
+        (150000, 256): "nn", (205000, 200): "nw", (255000, 200): "ww", (255000, 32): "nw", (200000, 4): "nw",
+    }
+    got = child(f"""
+ctx, out = wg.Context(0), []
+for m, n in {list(shapes)}:
+    for gemv in (ctx.sgemv, ctx.dgemv):
+        log, error = calls(lambda: gemv(0, m, n, 1.0, P, m, P, 1, 0.0, P, 1))
+        assert error is None, error
+        out.append(next(line.split() for line in log if "gemv_n_kernel" in line))
+print(json.dumps(out))
+""")
+    kinds = {}
+    for k, (m, n) in enumerate(shapes):
+        for line in got[2 * k:2 * k + 2]:
+            across, splits, threads = int(line[1]), int(line[2]), int(line[4])
+            narrow = threads == 512
+            kinds[m, n] = kinds.get((m, n), "") + ("n" if narrow else "w")
+            rows = 256 if narrow else 1024
+            assert (across - 1) * rows < m <= across * rows
+            if narrow and across <= 256:
+                assert across * splits <= 256, (m, n, across, splits)
+    assert kinds == shapes

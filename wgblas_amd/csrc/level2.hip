@@ -51,8 +51,8 @@ constexpr int64_t kShortColsRows = 4096;
 constexpr int kStepN = 8;
 constexpr int kTargetBlocksN = 256;
 constexpr int kMinColsN = 256;
-// Where those blocks would be fewer than the target (below 8192 x 8192):
-// blocks of 256 rows whose kColWaves waves share at least kMinColsNarrow
+// Beside them, for small matrices and few rows (plan_n): blocks of 256 rows whose
+// kColWaves waves share at least kMinColsNarrow
 // columns, partial sums added in LDS. 4096^2, fp32: 64 wide blocks 38.2 us, 256
 // narrow ones 12.9 (5.2 TB/s; 4 waves 16.4); fp64 70.2 and 27.1. Splits of at
 // least 64 / 128 / 256 columns: fp32 512^2 6.9 / 6.6 / 8.6 us, fp64 8.7 / 10.2 /
@@ -1067,6 +1067,53 @@ int trmv(wgb_ctx *ctx, int uplo, int trans, int diag, int64_t n, const T *A, int
   return WGB_OK;
 }
 
+int64_t split_count(int64_t want, int64_t most) {
+  if (want > most) want = most;
+  if (want > 65535) want = 65535;  // grid y limit
+  return want < 1 ? 1 : want;
+}
+
+// The N form's blocks: narrow (256 rows, the columns shared by kColWaves waves)
+// or wide (1024 rows), how many side by side, and columns per split.
+//
+// Narrow: at most one block per CU where one per 256 rows is not more already
+// (a few more put two on some CUs, which the rest waits for: dgemv 15000 x 4000
+// in 59 x 5 blocks 127 us, in 59 x 4 94); whole steps for every wave.
+//
+// Either kind reads at about the same rate per CU, so the one that leaves the
+// busiest CU the smaller part of A (fp64: by 1/64) is the faster one, while the wide ones are
+// fewer than the CUs and hold kMinColsN columns or fewer (narrow / wide, us):
+// dgemv 1024 x 57000 88 / 92, 65000 100 / 98, 964 x 61000 102 / 94, 25000 x 2304
+// 100 / 91, 50000 x 768 62 / 82, 230000 x 200 70 / 66. In fp32 a wide block of
+// fewer rows takes as long (sgemv 800 x 65000 37 / 46) and the CUs keep several
+// narrow blocks apiece busy, up to 15/16 of the wide ones' rows (205000 x 200 31 /
+// 33, 255000 x 200 41 / 37) or over few columns (255000 x 32 7.7 / 8.9). Up to
+// 512 rows half of a wide block's waves and more would have none (sgemv 250 x
+// 70000 18 / 42, dgemv 512 x 160000 121 / 160).
+struct PlanN {
+  bool narrow;
+  int64_t blocks, per;
+};
+template <typename T>
+PlanN plan_n(int64_t m, int64_t n) {
+  const int64_t cus = kTargetBlocksN, unit = kColWaves * kStepN;
+  PlanN wide = {false, cdiv(m, 4 * kThreads), 0}, narrow = {true, cdiv(m, 256), 0};
+  wide.per = cdiv(n, split_count(cdiv(cus, wide.blocks), cdiv(n, kMinColsN)));
+  narrow.per = cdiv(cdiv(n, split_count(cus / narrow.blocks, cdiv(n, kMinColsNarrow))), unit) * unit;
+  if (m <= 512) return narrow;
+  if (wide.blocks * cdiv(n, kMinColsN) >= cus) return wide;
+  const int64_t cols = narrow.per < n ? narrow.per : n;
+  const int64_t rounds = cdiv(narrow.blocks * cdiv(n, narrow.per), cus);
+  bool better;
+  if (sizeof(T) == 8)
+    better = 64 * rounds * cols * 256 < 63 * wide.per * (m < 4 * kThreads ? m : 4 * kThreads);
+  else if (rounds == 1)
+    better = cols * 256 <= wide.per * 4 * kThreads;
+  else
+    better = n <= kMinColsN / 2 || 16 * narrow.blocks < 15 * 4 * cus;
+  return better ? narrow : wide;
+}
+
 // sgemv / dgemv on the kernels above. dgemv keeps reference BLAS's quick
 // return for alpha == 0 with beta == 1 (src/dgemv/dgemv.mjs:126: no
 // kernel, y untouched bit for bit); sgemv times an empty span there, as
@@ -1103,22 +1150,12 @@ int gemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, T alpha, const T *A, int
     return WGB_OK;
   }
   // blocks along the output; split the contraction dimension until about
-  // the target block count streams A (N: >= kMinColsN columns per split; T: >= 256
+  // the target block count streams A (N: plan_n; T: >= 256
   // rows, a multiple of 256 so every split starts aligned)
   const int cpw = m <= kShortColsRows ? kColsPerWaveShort : kColsPerWave;  // T form
-  // N form: where 1024-row blocks of at least kMinColsN columns are fewer than
-  // the target, blocks of 256 rows whose waves share the columns
-  const bool narrow = nt && cdiv(m, 4 * kThreads) * cdiv(n, kMinColsN) < kTargetBlocksN;
-  const int64_t bx = nt ? cdiv(m, narrow ? 256 : 4 * kThreads) : cdiv(cdiv(n, cpw), kThreads / 64);
-  const int64_t target = nt ? kTargetBlocksN : kTargetBlocks;
-  int64_t want = bx >= target ? 1 : cdiv(target, bx);
-  const int64_t most = nt ? cdiv(n, narrow ? kMinColsNarrow : kMinColsN) : cdiv(m, 256);
-  if (want > most) want = most;
-  if (want > 65535) want = 65535;  // grid y limit
-  if (want < 1) want = 1;
-  // (narrow: whole steps for every wave)
-  const int64_t unit = narrow ? kColWaves * kStepN : 1;
-  const int64_t per = nt ? cdiv(cdiv(n, want), unit) * unit : cdiv(cdiv(m, want), 256) * 256;
+  const PlanN plan = nt ? plan_n<T>(m, n) : PlanN{};
+  const int64_t bx = nt ? plan.blocks : cdiv(cdiv(n, cpw), kThreads / 64);
+  const int64_t per = nt ? plan.per : cdiv(cdiv(m, split_count(cdiv(kTargetBlocks, bx), cdiv(m, 256))), 256) * 256;
   const int64_t splits = nt ? cdiv(n, per) : cdiv(m, per);
   T *part = nullptr;
   if (splits > 1) {
@@ -1134,7 +1171,7 @@ int gemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, T alpha, const T *A, int
     auto launch = [&](auto kern, int threads) {
       kern<<<grid, threads, 0, ctx->stream>>>(m, n, A, lda, x, incx, per, part, alpha, beta, y, incy);
     };
-    if (narrow)
+    if (plan.narrow)
       launch(vec == kVecA   ? gemv_n_kernel<T, kVecA, 1, kColWaves>
              : vec == kVecU ? gemv_n_kernel<T, kVecU, 1, kColWaves>
                             : gemv_n_kernel<T, kElems, 1, kColWaves>,
