@@ -104,6 +104,16 @@ print(json.dumps(out))
         assert launches == ([False, True] if two else [False]), (capturing, n, launches)
 
 
+def test_a_captured_host_result_ends_the_capture(child):
+    """The host forms do not ask whether the stream is capturing: their wait for it is refused there."""
+    got = child("""
+ctx = wg.Context(0)
+runtime.standin_capture(1)
+print(json.dumps(calls(lambda: ctx.sasum(100_003, P, 1))))
+""")
+    assert got[0][-1] == "synchronize" and "status -2" in got[1], got
+
+
 def test_a_missing_result_clears_the_arrival_count(child):
     """The next call starts from 0 whatever kept this one from storing its result."""
     got = child("""
@@ -125,13 +135,13 @@ def test_the_result_slot_is_coherent_memory(child):
 
 
 def test_reductions_fold_in_the_same_launch_only_where_that_is_no_slower(child):
-    """Sums of one word up to 256 first-pass blocks of 4096 elements, folds of more words and
-    strided reads up to 192, strided reads of 8-byte elements up to 128."""
+    """Sums of one word up to 256 first-pass blocks of 4096 elements, folds of up to 16 bytes and
+    strided reads up to 192, larger folds and strided reads of 8-byte elements up to 112."""
     got = child("""
 ctx, out = wg.Context(0), []
 for name, two, blocks, inc in (("sdot", 1, 256, 1), ("ddot", 1, 256, 1), ("dasum", 0, 256, 1), ("snrm2", 0, 192, 1),
-                               ("dnrm2", 0, 192, 1), ("isamax", 0, 192, 1), ("idamax", 0, 192, 1),
-                               ("ddot", 1, 128, 5), ("sasum", 0, 192, 7), ("dnrm2", 0, 128, 6)):
+                               ("dnrm2", 0, 112, 1), ("isamax", 0, 192, 1), ("idamax", 0, 192, 1),
+                               ("ddot", 1, 112, 5), ("sasum", 0, 192, 7), ("dnrm2", 0, 112, 6)):
     for n in (blocks * 4096, blocks * 4096 + 1):
         args = (n, P, inc, P, inc, P) if two else (n, P, inc, P)
         log, error = calls(lambda: getattr(ctx, name + "_dev")(*args))
@@ -198,3 +208,18 @@ print(json.dumps(out))
             if narrow and across <= 256:
                 assert across * splits <= 256, (m, n, across, splits)
     assert kinds == shapes
+
+
+def test_long_reductions_keep_the_plain_remainder_loop(child):
+    """Where a thread has more than a few steps, taking what kUnroll leaves over four at a time (and
+    the folding code beside it) was slower than one at a time."""
+    got = child("""
+ctx, out = wg.Context(0), []
+for name, n in (("isamax", 24_000_000), ("isamax", 32_000_000), ("idamax", 20_000_000), ("idamax", 24_000_000),
+                ("isamax", 1), ("isamax", 1_000_000), ("idamax", 1_000_000)):
+    log, error = calls(lambda: getattr(ctx, name + "_dev")(n, P, 1, P))
+    assert error is None, error
+    out.append(next(line.split()[-1] for line in log if "reduce_vec" in line))
+print(json.dumps(out))
+""")
+    assert ["Lb1E" in name for name in got] == [True, False, True, False, True, True, True], got

@@ -65,19 +65,26 @@ constexpr int kThreads = 256;
 // the box's read roof measured by roof_probe: 7.1 TB/s).
 constexpr int kUnroll = 16;
 constexpr int kTail = 4;  // loads in flight over what is left of a range
+// Elements per thread up to which reduce_vec takes kTail of them at a time where
+// kUnroll are too many (and may fold): us a call with / without, isamax 16 777 216
+// floats 14.5 / 15.8, 24 000 000 19.6 / 19.7, 32 328 320 25.9 / 24.1, 48 000 000
+// 33.4 / 31.9; dnrm2 6 000 000 doubles 13.0 / 13.8, 20 000 000 29.2 / 30.2,
+// 24 000 000 36.3 / 34.5.
+constexpr int kShortShare4 = 24, kShortShare8 = 20;
 constexpr int64_t kElemsPerBlockMin = 4096;
 // Up to this many first-pass blocks the last one to arrive folds (one launch).
 // The arrivals serialise on one word, about 10 ns each, and the fold comes
 // after them, against a second launch that costs about 2 us where launches are
 // what a call waits for and little where the read hides it. One launch / two,
-// us a call, results left in device memory, on two boxes whose launches differ:
+// us a call, results left in device memory, on two hosts whose launches differ:
 // sdot 256 blocks 6.4 / 6.6, dasum 256 7.1 / 7.7; folds of more than one word
 // cost more: isamax 192 blocks 6.4 / 6.3 and 6.4 / 7.3, 224 6.8 / 6.3 and 6.8 /
-// 7.3, dnrm2 192 7.8 / 7.8, 224 8.2 / 7.8; strided reads are longer: sdot, stride
-// 5, 192 blocks 6.8 / 7.2, 245 9.9 / 9.2, ddot 128 9.6 / 9.7, 160 11.4 / 11.0.
+// 7.3, dnrm2 (32 bytes) 128 blocks 6.5 / 6.4 and 6.9 / 7.6, 160 7.0 / 6.4 and 7.2 /
+// 7.9; strided reads are longer: sdot, stride 5, 192 blocks 6.8 / 7.2, 245 9.9 /
+// 9.2, ddot 128 9.6 / 9.2, 160 11.4 / 11.0.
 constexpr int kMaxFusedBlocks = 256;
-constexpr int kMaxFusedDear = 192;      // more than one word to fold, or a strided read
-constexpr int kMaxFusedStrided8 = 128;  // a strided read of 8-byte elements
+constexpr int kMaxFusedDear = 192;    // more than 8 bytes to fold, or a strided read
+constexpr int kMaxFusedDearer = 112;  // more than 16 bytes, or a strided read of 8-byte elements
 
 // snrm2 thresholds and scales (powers of two): src/shaders/snrm2.wgsl:33-36.
 constexpr float kTsml = 0x1p-63f;
@@ -505,18 +512,18 @@ __device__ __forceinline__ P load_partial(const P *slot) {
   return p;
 }
 
-// A block's partial goes to its slot. With at most kMaxFusedBlocks blocks
-// (`out` given) the block that arrives last folds them all in the same
+// A block's partial goes to its slot. With few blocks (MAY_FUSE, and
+// `out` given) the block that arrives last folds them all in the same
 // launch, in fold_kernel's order; otherwise stage 2 (fold_kernel) does.
 // The arrival is ordered after the partial by waiting for the stores
 // (s_waitcnt vmcnt(0)): a release fence at agent scope would write back the
 // XCD's L2 in every block (~90 us per 2048-block launch on MI355X).
 // The last block sets the counter back to 0 for the stream's next launch
 // (captured launches of several blocks never count: fuse_fold).
-template <class Op>
+template <class Op, bool MAY_FUSE = true>
 __device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Partial *partials,
                                        uint32_t *arrived, Output<Op> out) {
-  if (!out.ptr) {
+  if (!MAY_FUSE || !out.ptr) {
     if (threadIdx.x == 0) partials[blockIdx.x] = p;
     return;
   }
@@ -532,9 +539,8 @@ __device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Part
   __syncthreads();
   if (!last) return;
   if (gridDim.x > 1) {
+    static_assert(kMaxFusedBlocks <= kThreads, "one partial a thread");
     p = threadIdx.x < gridDim.x ? load_partial(partials + threadIdx.x) : Op::identity();
-    for (uint32_t i = threadIdx.x + kThreads; i < gridDim.x; i += kThreads)
-      p = Op::merge(p, load_partial(partials + i));
     p = block_merge<Op>(p);
   }
   if (threadIdx.x == 0) {
@@ -545,7 +551,7 @@ __device__ __forceinline__ void finish(typename Op::Partial p, typename Op::Part
 
 // Unit-stride, 16-byte-aligned operands: 16-byte non-temporal loads,
 // kUnroll of them in flight per lane per input.
-template <class Op>
+template <class Op, bool SHORT>
 __global__ __launch_bounds__(kThreads) void reduce_vec(const typename Op::Elem *__restrict__ x,
                                                        const typename Op::Elem *__restrict__ y, int64_t n,
                                                        typename Op::Partial *__restrict__ partials,
@@ -570,7 +576,7 @@ __global__ __launch_bounds__(kThreads) void reduce_vec(const typename Op::Elem *
     for (int u = 0; u < kUnroll; ++u) Op::addv(s, a[u], b[u], W * (q + u * kThreads));
   }
   // what is left (a short vector's whole share), kTail loads in flight
-  for (; q + (kTail - 1) * kThreads < end; q += kTail * kThreads) {
+  for (; SHORT && q + (kTail - 1) * kThreads < end; q += kTail * kThreads) {
     V a[kTail], b[kTail];
 #pragma unroll
     for (int u = 0; u < kTail; ++u) {
@@ -588,7 +594,7 @@ __global__ __launch_bounds__(kThreads) void reduce_vec(const typename Op::Elem *
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
     for (int64_t i = nv * W; i < n; ++i)
       Op::add1(s, x[i], Op::NIN == 2 ? y[i] : (typename Op::Elem)0, i, 0);
-  finish<Op>(block_merge<Op>(Op::finish(s)), partials, arrived, out);
+  finish<Op, SHORT>(block_merge<Op>(Op::finish(s)), partials, arrived, out);
 }
 
 // Whether Op has add_kept (a vector of which some elements are kept).
@@ -817,10 +823,11 @@ void *arrival_counter(wgb_ctx *ctx) {
 // launch. The context's stream orders the launches that count arrivals, but a
 // captured graph may be replayed on another stream, beside them: a count that
 // two launches share would stay off zero for every later call. Captured
-// launches therefore keep none (one block has nothing to count).
-int fuse_fold(wgb_ctx *ctx, int G, int most, bool *fuse) {
+// launches therefore keep none (one block has nothing to count; a host-result
+// call cannot be captured: its wait for the stream ends the capture).
+int fuse_fold(wgb_ctx *ctx, int G, int most, bool host, bool *fuse) {
   *fuse = G <= most;
-  if (!*fuse || G == 1) return WGB_OK;
+  if (!*fuse || host || G == 1) return WGB_OK;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   WGB_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &status));
   *fuse = status == hipStreamCaptureStatusNone;
@@ -843,14 +850,18 @@ int launch_reduce(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t i
   // G from the span, not n, where each block reads a span range.
   const int G = reduce_blocks(by_span ? span : n);
   const bool strided = !vec && !by_span && (incx > 1 || (Op::NIN == 2 && incy > 1));
-  const int most = strided && sizeof(typename Op::Elem) == 8 ? kMaxFusedStrided8
-                   : strided || sizeof(typename Op::Partial) > 8 ? kMaxFusedDear : kMaxFusedBlocks;
+  const size_t fold = sizeof(typename Op::Partial);
+  const int most = fold > 16 || (strided && sizeof(typename Op::Elem) == 8) ? kMaxFusedDearer
+                   : fold > 8 || strided                                    ? kMaxFusedDear
+                                                                            : kMaxFusedBlocks;
   bool fuse = false;
   int st;
-  if ((st = fuse_fold(ctx, G, most, &fuse))) return st;
+  if ((st = fuse_fold(ctx, G, most, out.seq != 0, &fuse))) return st;
   const Output<Op> fused = fuse ? out : Output<Op>{nullptr, 0};
-  if (vec)
-    reduce_vec<Op><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
+  if (vec && n <= (int64_t)G * kThreads * (sizeof(typename Op::Elem) == 4 ? kShortShare4 : kShortShare8))
+    reduce_vec<Op, true><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
+  else if (vec)
+    reduce_vec<Op, false><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
   else if (by_span && incx == 2)
     reduce_span<Op, 2><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
   else if (by_span && incx == 3)
