@@ -7,7 +7,9 @@
     and matrices whose columns are aligned (lda % 4 == 0) or not; the split of
     gemv's columns over a block's waves, and a triangle's runs that end inside
     a 1024-row chunk;
-  * gemm: k-tiles shared by 2 or 4 groups of waves, with unequal shares.
+  * gemm: k-tiles shared by 2 or 4 groups of waves, with equal and unequal
+    shares (the group count that the shapes are there for is checked on the CPU
+    too, against the kernel that the library launches).
 
 References are numpy in float64 (whole-number data where the sums are exact in
 either precision, so that those results compare exactly)."""
@@ -53,7 +55,7 @@ def _triangle(A, uplo, unit=False):
 
 
 @pytest.mark.parametrize("prefix,dtype", [("s", np.float32), ("d", np.float64)])
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 257, 1023, 1025, 2050, 3333])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 257, 1023, 1025, 2050, 3333, 5125])
 @pytest.mark.parametrize("pad", [0, 3])
 def test_level2_edges(ctx, prefix, dtype, n, pad):
     rng = np.random.default_rng(10 * n + pad)
@@ -116,18 +118,66 @@ def test_gemv_wide_blocks(ctx, prefix, dtype, m, n, lda):
             buf.free()
 
 
+def _k_groups(m, n, k, uplo=0):
+    """How many groups of waves share a 64 x 64 tile's k-tiles of 32 on 256 CUs."""
+    tm, tn = -(-m // 64), -(-n // 64)
+    assert not uplo or m == n
+    tiles = tm * (tm + 1) // 2 if uplo else tm * tn
+    ktiles = -(-k // 32)
+    if tiles <= 256:
+        return 4 if ktiles >= 64 else 2 if ktiles >= 16 else 1
+    return 2 if tiles <= 512 and ktiles >= 64 else 1
+
+
+# (m, n, k, padding of every leading dimension, groups)
+K_GROUPS = [
+    (1024, 1024, 545, 0, 2),  # 18 k-tiles, 9 each, whole tiles, a partial last k-tile
+    (1000, 1001, 1040, 0, 2),  # 33: 17 and 16, edge tiles
+    (1024, 900, 549, 4, 2),  # 18, an edge in n, a last k-tile of 5
+    (640, 640, 2049, 0, 4),  # 65: 17 16 16 16, one column in the last k-tile
+    (500, 700, 2113, 1, 4),  # 67: 17 17 17 16, edges, leading dimensions that are no multiple of 4
+    (640, 640, 2112, 0, 4),  # 66: 17 17 16 16, whole k-tiles
+    (640, 577, 2048, 64, 4),  # 64, equal shares
+    (1500, 1000, 2081, 0, 2),  # 384 tiles, 66 k-tiles
+    (1280, 1600, 2112, 1, 2),  # 500 tiles, 33 each
+]
+# just outside the rule: too few k-tiles, or more tiles than CUs
+ONE_GROUP = [(1024, 1024, 256, 0, 1), (1000, 1025, 263, 0, 1), (900, 1100, 1090, 0, 1), (1500, 1400, 301, 0, 1),
+             (2048, 1024, 320, 0, 1)]
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("m,n,k", [(1024, 1024, 256), (1000, 1025, 263), (1024, 1024, 545), (900, 1100, 1090),
-                                   (1500, 1400, 301), (2048, 1024, 320)])
-def test_sgemm_k_groups(ctx, ta, tb, m, n, k):
-    """8 k-tiles of 32 and more: equal and unequal shares, a partial last k-tile, edge tiles. Exact: whole
-    numbers, |sums| <= 49 k + 1 < 2^24."""
+@pytest.mark.parametrize("m,n,k,pad,groups", K_GROUPS + ONE_GROUP)
+def test_sgemm_k_groups(ctx, ta, tb, m, n, k, pad, groups):
+    """Equal and unequal shares, edge tiles, partial last k-tiles, operands at any alignment. Exact: whole numbers,
+    |sums| <= 49 k + 7 < 2^24."""
+    assert _k_groups(m, n, k) == groups
     rng = np.random.default_rng(m + n + k)
-    A, B = _ints(rng, (m, k) if ta else (k, m), np.float32), _ints(rng, (k, n) if tb else (n, k), np.float32)
-    C = _ints(rng, (n, m), np.float32)
+    rows_a, rows_b = (k if ta else m) + pad, (n if tb else k) + pad
+    A, B = _ints(rng, (m if ta else k, rows_a), np.float32), _ints(rng, (k if tb else n, rows_b), np.float32)
+    C = _ints(rng, (n, m + pad), np.float32)
     dC = ctx.upload(C)
-    ctx.sgemm(ta, tb, m, n, k, 1.0, ctx.upload(A), k if ta else m, ctx.upload(B), n if tb else k, -1.0, dC, m)
+    ctx.sgemm(ta, tb, m, n, k, 1.0, ctx.upload(A), rows_a, ctx.upload(B), rows_b, -1.0, dC, m + pad)
+    A, B = A[:, :k if ta else m], B[:, :n if tb else k]
     opA = A if ta else A.T  # m x k
     opB = B if tb else B.T  # k x n
-    want = (opA.astype(np.float64) @ opB.astype(np.float64)).T - C
-    assert np.array_equal(dC.to_host().reshape(n, m), want)
+    want = C.astype(np.float64)
+    want[:, :m] = (opA.astype(np.float64) @ opB.astype(np.float64)).T - C[:, :m]
+    assert np.array_equal(dC.to_host().reshape(n, m + pad), want)
+
+
+@pytest.mark.parametrize("uplo", [1, 2])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("n,k,groups", [(1001, 1040, 2), (700, 2113, 4)])
+def test_sgemmtr_k_groups(ctx, uplo, ta, tb, n, k, groups):
+    """The same on a triangle's tiles; the other triangle is untouched."""
+    assert _k_groups(n, n, k, uplo) == groups
+    rng = np.random.default_rng(n + k)
+    A, B = _ints(rng, (n, k) if ta else (k, n), np.float32), _ints(rng, (k, n) if tb else (n, k), np.float32)
+    C = _ints(rng, (n, n), np.float32)
+    dC = ctx.upload(C)
+    ctx.sgemmtr(uplo, ta, tb, n, n, k, 1.0, ctx.upload(A), k if ta else n, ctx.upload(B), n if tb else k, -1.0, dC, n)
+    opA, opB = (A if ta else A.T).astype(np.float64), (B if tb else B.T).astype(np.float64)
+    keep = np.tri(n, dtype=bool) if uplo == 1 else np.tri(n, dtype=bool).T
+    want = np.where(keep.T, (opA @ opB).T - C, C)
+    assert np.array_equal(dC.to_host().reshape(n, n), want)

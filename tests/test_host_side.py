@@ -223,3 +223,61 @@ for name, n in (("isamax", 24_000_000), ("isamax", 32_000_000), ("idamax", 20_00
 print(json.dumps(out))
 """)
     assert ["Lb1E" in name for name in got] == [True, False, True, False, True, True, True], got
+
+
+def test_sgemm_k_groups_are_reached(child):
+    """The shapes of the k-group tests launch the kernel that they are there for, in every layout; one k-tile or
+    one tile fewer or more than the rule's lines does not."""
+    from tests.test_gpu_dispatch_edges import K_GROUPS, ONE_GROUP
+
+    assert {case[-1] for case in K_GROUPS} == {2, 4}
+    got = child(f"""
+out = []
+ctx = wg.Context(0)
+for m, n, k, pad, groups in {K_GROUPS + ONE_GROUP}:
+    for ta in (0, 1):
+        for tb in (0, 1):
+            log, error = calls(lambda: ctx.sgemm(ta, tb, m, n, k, 1.0, P, (k if ta else m) + pad, P, (n if tb else k) + pad,
+                                                 -1.0, P, m + pad))
+            out.append([groups, log[-1].split()])
+for n, k, groups in ((1001, 1040, 2), (700, 2113, 4)):
+    log, error = calls(lambda: ctx.sgemmtr(1, 0, 0, n, n, k, 1.0, P, n, P, k, -1.0, P, n))
+    out.append([groups, log[-1].split()])
+for m, n, k in ((1024, 1024, 480), (1024, 1088, 1000), (2048, 1088, 2048), (2048, 1024, 2016)):
+    log, error = calls(lambda: ctx.sgemm(0, 1, m, n, k, 1.0, P, m, P, n, -1.0, P, m))
+    out.append([1, log[-1].split()])
+print(json.dumps(out))
+""")
+    for groups, (_, _, _, _, threads, name) in got:
+        assert int(threads) == 256 * groups, (groups, threads, name)
+        assert ("gemm_kgroup_kernelILi%dE" % groups in name) == (groups > 1), (groups, name)
+
+
+@pytest.mark.parametrize("prefix,size", [("s", 4), ("d", 8)])
+def test_symv_plan(child, prefix, size):
+    """The runs of symv / trmv: at most 512 columns (the LDS of their sums), the workspace large enough for
+    every chunk's row slots and column slots, and all columns covered."""
+    got = child(f"""
+out = []
+for n in list(range(1, 70)) + [1023, 1024, 1025, 2049, 4096, 5120, 5121, 6001, 8191, 8192, 16383, 22528, 23000, 32769, 65536]:
+    for uplo in (1, 2):
+        ctx = wg.Context(0)  # a workspace of its own
+        log, error = calls(lambda: ctx.{prefix}symv(uplo, n, 1.0, P, n, P, 1, 0.0, P, 1))
+        assert error is None, error
+        ws = [int(line.split()[1]) for line in log if line.startswith("malloc")]
+        blocks = next(int(line.split()[1]) for line in log if "symv_kernel" in line)
+        out.append([n, uplo, blocks, ws])
+        ctx.close()
+print(json.dumps(out))
+""")
+    for n, uplo, blocks, ws in got:
+        chunks = -(-n // 1024)
+        n8 = -(-n // 8) * 8
+        columns = [min((r + 1) * 1024, n8) if uplo == 1 else n8 - r * 1024 for r in range(chunks)]
+        # the run is not in the log: some multiple of 8 that gives this many blocks
+        total = sum(columns)
+        runs = [run for run in range(8, 513, 8) if -(-total // run) == blocks]
+        assert runs, (n, uplo, blocks)
+        starts = [sum(columns[:r]) for r in range(chunks)]
+        need = min(max((s + c - 1) // run - s // run + 1 for s, c in zip(starts, columns)) for run in runs)
+        assert len(ws) == 1 and ws[0] >= (need + chunks) * n * size, (n, uplo, blocks, ws)
