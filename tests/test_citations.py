@@ -68,7 +68,11 @@ def _resolve(cited, ref_names, own_names):
     return []
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference checkout not present")
+def _reference_present():
+    return os.path.isdir(REF) and bool(os.listdir(REF))
+
+
+@pytest.mark.skipif(not _reference_present(), reason="reference checkout not present")
 def test_every_citation_is_in_range():
     ref_names, own_names = _index(REF), _index(ROOT)
     bad = []
@@ -132,7 +136,7 @@ def _named_in_range(pattern, cites, ref_names, own_names):
     return in_file, in_range
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference checkout not present")
+@pytest.mark.skipif(not _reference_present(), reason="reference checkout not present")
 def test_cited_range_holds_the_named_symbol():
     """Where a citation names what it cites — a symbol or a message right
     before the parenthesised citations, or the definition that a doc comment
