@@ -362,8 +362,8 @@ int wgb_dsymv(wgb_ctx *ctx, int uplo, int64_t n, double alpha, const double *A,
  * incy > 0; y is written, never read, and must not overlap A or x. The
  * WGB_NO_TRANS form skips a column whose x entry is zero (reference BLAS's
  * column form), the transposed one takes every term. One pass over the
- * triangle (row or column sums of 1024 x 128 blocks), then a fixed-order
- * fold (deterministic). Replaces strmv (src/strmv/strmv.mjs:20-259,
+ * triangle (row or column sums of runs of up to 512 columns of 1024 rows),
+ * then a fixed-order fold (deterministic). Replaces strmv (src/strmv/strmv.mjs:20-259,
  * src/shaders/strmv.wgsl, strmv_t.wgsl, reduce_partials.wgsl). */
 int wgb_strmv(wgb_ctx *ctx, int uplo, int trans, int diag, int64_t n,
               const float *A, int64_t lda, const float *x, int64_t incx,
@@ -385,10 +385,14 @@ int wgb_dgemv(wgb_ctx *ctx, int trans, int64_t m, int64_t n, double alpha,
 
 /* ---- level 1 reductions --------------------------------------------------- */
 /* n <= 0 returns 0 (index -1) without touching the device. incx, incy must be
- * positive. The host-result forms block until the value is on the host; the
- * `_dev` forms write the result to device memory and return without
- * synchronising. Both run a fixed two-pass reduction whose summation order
- * depends only on n, so results are reproducible run to run.
+ * positive. The host-result forms block until the value is on the host: the
+ * operands have been read and earlier work of the stream is done, but the
+ * stream itself is not drained (wgb_synchronize does that); a stream that ends
+ * without the value gives WGB_ERR_HIP. The `_dev` forms write the result to
+ * device memory and return without synchronising. Both fold per-block sums
+ * (in the same launch for short vectors) in an order that depends only on n, the
+ * strides and the operands' 16-byte alignment, so results are reproducible run
+ * to run.
  *
  * The reductions of one context share its scratch memory, in the order of its
  * stream. Under capture the `_dev` forms record kernels only; a graph that

@@ -40,7 +40,7 @@ constexpr int kThreads = 256;
 constexpr int kColsPerWave = 8;
 constexpr int kColsPerWaveShort = 4;
 constexpr int64_t kShortColsRows = 4096;
-// N form: columns loaded per step, 1024-row groups per block, the blocks
+// N form: columns loaded per step, and for blocks of 1024 rows the number
 // aimed for and the fewest columns per split. Measured on MI355X over
 // 2048 x 65536, 8192^2, 16384^2, 32768^2 and 65536 x 2048 (sweep of 1 or 2
 // groups, 256 / 512 / 1024 target blocks, 256 or 512 columns): one group,

@@ -904,7 +904,7 @@ int reduce_to_device(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_
 
 // Waits for call `seq`'s number in the host slot (four reductions of 100 003
 // floats, host results: copy command and stream wait 76.2 us, stream wait alone
-// 65.4, this 45.9): read directly for as long as a
+// 65.4, this 46.5): read directly for as long as a
 // short reduction takes, then by waiting for the stream, whose own wait costs
 // several us more. The slot keeps an earlier call's value until this one's
 // arrives, so a stream that ends without it is an error; the count of arrivals
