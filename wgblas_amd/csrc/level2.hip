@@ -444,6 +444,7 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
     int64_t m, int64_t n, T alpha, const T *__restrict__ x, int64_t incx, const T *__restrict__ y,
     int64_t incy, T *__restrict__ A, int64_t lda, int64_t cpb) {
   typedef vec4<T> f4;
+  constexpr int kVecCut = 3;
   // columns [j0, j1) of the 1024 rows from r0 on
   auto chunk = [&](const int64_t r0, int64_t j0, int64_t j1) {
   const int64_t ib = r0 + 4 * threadIdx.x;  // the lane's own rows start here
@@ -475,7 +476,8 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
     }
   };
   // MODE: how the wave accesses A, whole vectors with no per-lane branch
-  // between the stores (kVecA: non-temporal), or kElems for a wave with fewer
+  // between the stores (kVecA: non-temporal; kVecCut: in a chunk that m cuts, as
+  // kVecU), or kElems for a wave with fewer
   // than 4 rows (its loads are still whole vectors where m >= 4) or a matrix with
   // fewer. A lane whose rows cross m updates the last 4 rows of its wave, as its
   // neighbours in the same instructions do: the rows they share get the same
@@ -506,10 +508,17 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
         }
       }
       if (FULL || (VEC && lo == 0)) {
-        if constexpr (MODE == kVecA)
+        if constexpr (MODE == kVecA) {
           __builtin_nontemporal_store(v, reinterpret_cast<vec4u<T> *>(col + i0));
-        else
+        } else if constexpr (MODE == kVecCut) {
+          // all of the column's vector is loaded before any part of it is stored:
+          // lanes that share rows must not read each other's results
+          T a = v[0], b = v[1], c = v[2], d = v[3];
+          asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : : "memory");
+          *reinterpret_cast<vec4u<T> *>(col + i0) = f4{a, b, c, d};
+        } else {
           *reinterpret_cast<vec4u<T> *>(col + i0) = v;
+        }
       } else {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -555,7 +564,7 @@ __global__ __launch_bounds__(kThreads) void rank_update_kernel(
     if (vectors && !cut)
       walk(std::integral_constant<int, VEC>{}, mask_tag, ja, jb);
     else if (vectors)
-      walk(std::integral_constant<int, VEC ? kVecU : kElems>{}, mask_tag, ja, jb);
+      walk(std::integral_constant<int, VEC ? kVecCut : kElems>{}, mask_tag, ja, jb);
     else
       walk(std::integral_constant<int, kElems>{}, mask_tag, ja, jb);
   };
