@@ -183,7 +183,7 @@ def test_gemv_blocks_by_the_busiest_cu(child):
         # the wide blocks fill the CUs
         (8192, 8192): "ww", (16384, 16384): "ww", (1025, 40000): "ww", (400000, 10): "ww",
         # splits that do not divide the CUs' work evenly
-        (15000, 4000): "ww", (25000, 2304): "ww", (1024, 57000): "nn", (1024, 65000): "nw",
+        (15000, 4000): "nw", (25000, 2304): "nw", (1024, 57000): "nn", (1024, 65000): "nw",
         (964, 61000): "nw", (800, 65000): "nw",
         # more than one narrow block per CU beside each other
         (150000, 256): "nn", (205000, 200): "nw", (255000, 200): "ww", (255000, 32): "nw", (200000, 4): "nw",

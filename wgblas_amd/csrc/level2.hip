@@ -1093,10 +1093,11 @@ int64_t split_count(int64_t want, int64_t most) {
 // busiest CU the smaller part of A (fp64: by 1/64) is the faster one, while the wide ones are
 // fewer than the CUs and hold kMinColsN columns or fewer (narrow / wide, us):
 // dgemv 1024 x 57000 88 / 92, 65000 100 / 98, 964 x 61000 102 / 94, 25000 x 2304
-// 100 / 91, 50000 x 768 62 / 82, 230000 x 200 70 / 66. In fp32 a wide block of
-// fewer rows takes as long (sgemv 800 x 65000 37 / 46) and the CUs keep several
-// narrow blocks apiece busy, up to 15/16 of the wide ones' rows (205000 x 200 31 /
-// 33, 255000 x 200 41 / 37) or over few columns (255000 x 32 7.7 / 8.9). Up to
+// 100 / 91, 50000 x 768 62 / 82, 230000 x 200 70 / 66. In fp32 the CUs read narrow
+// blocks faster, and a wide block of fewer rows takes as long (sgemv 15000 x 4352
+// 46 / 47, 25000 x 2304 41 / 45, 800 x 65000 37 / 46): narrow ones wherever they are
+// one per CU, else up to 15/16 of the wide ones' rows (205000 x 200 31 / 33,
+// 255000 x 200 41 / 37) or over few columns (255000 x 32 7.7 / 8.9). Up to
 // 512 rows half of a wide block's waves and more would have none (sgemv 250 x
 // 70000 18 / 42, dgemv 512 x 160000 121 / 160).
 struct PlanN {
@@ -1116,10 +1117,8 @@ PlanN plan_n(int64_t m, int64_t n) {
   bool better;
   if (sizeof(T) == 8)
     better = 64 * rounds * cols * 256 < 63 * wide.per * (m < 4 * kThreads ? m : 4 * kThreads);
-  else if (rounds == 1)
-    better = cols * 256 <= wide.per * 4 * kThreads;
   else
-    better = n <= kMinColsN / 2 || 16 * narrow.blocks < 15 * 4 * cus;
+    better = rounds == 1 || n <= kMinColsN / 2 || 16 * narrow.blocks < 15 * 4 * cus;
   return better ? narrow : wide;
 }
 
