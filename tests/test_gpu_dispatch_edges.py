@@ -118,6 +118,28 @@ def test_gemv_wide_blocks(ctx, prefix, dtype, m, n, lda):
             buf.free()
 
 
+@pytest.mark.parametrize("prefix,dtype", [("s", np.float32), ("d", np.float64)])
+@pytest.mark.parametrize("lda", [8192, 8195])
+def test_gemv_sums_a_step_before_it_adds_it(ctx, prefix, dtype, lda):
+    """A 1 followed by products that are each too small to change it: with u half an ulp of 1, one chain over the
+    256 columns of the first split loses 255 * 0.99 u. A chain of 8 products a step (u each), an add for each of
+    256 / 8 steps, one for each of the 32 splits and 8 for alpha, beta
+    and the fold stay within 80 u of 1."""
+    m = n = 8192
+    u = np.finfo(dtype).eps / 2
+    A = np.full((n, lda), 0.99 * u, dtype)
+    A[0] = 1
+    dA, dx, dy = ctx.upload(A), ctx.upload(np.ones(n, dtype)), ctx.upload(np.zeros(m, dtype))
+    try:
+        getattr(ctx, prefix + "gemv")(0, m, n, 1.0, dA, lda, dx, 1, 0.0, dy, 1)
+        # differences from 1 are exact; what is wanted of them is (n - 1) products
+        over = (dy.to_host() - dtype(1)).astype(np.float64)
+        assert np.abs(over - (n - 1) * float(A[1, 0])).max() <= 80 * u
+    finally:
+        for buf in (dA, dx, dy):
+            buf.free()
+
+
 def _k_groups(m, n, k, uplo=0):
     """How many groups of waves share a 64 x 64 tile's k-tiles of 32 on 256 CUs."""
     tm, tn = -(-m // 64), -(-n // 64)

@@ -216,13 +216,21 @@ __global__ __launch_bounds__(64 * RW *CW) void gemv_n_kernel(int64_t m, int64_t 
 #pragma unroll
         for (int q = 0; q < 4; ++q) av[c][q] = held(av[c][q]);
     }
+    // The step's own sums, then one add each: a chain of kStepN products and
+    // per / kStepN adds in place of one of per products. Error against 64 bits
+    // (sgemv) and a compensated sum (dgemv), without / with: sgemv 8100 x 7900
+    // 2.1e-7 / 1.2e-7, dgemv 15000 x 4000 5.4e-16 / 2.7e-16; no time in sgemv,
+    // 0.4 % in dgemv (geometric means of 117 timings each).
+    T sum[4] = {(T)0, (T)0, (T)0, (T)0};
 #pragma unroll
     for (int c = 0; c < kStepN; ++c) {
       if (xv[c] != (T)0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = fma(av[c][q], xv[c], acc[q]);
+        for (int q = 0; q < 4; ++q) sum[q] = fma(av[c][q], xv[c], sum[q]);
       }
     }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] += sum[q];
   };
   auto walk = [&](auto whole_tag) {
     for (; j + kStepN <= j1; j += kStepN) step(std::false_type{}, whole_tag);
