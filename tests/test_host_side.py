@@ -211,18 +211,21 @@ print(json.dumps(out))
 
 
 def test_long_reductions_keep_the_plain_remainder_loop(child):
-    """Where a thread has more than a few steps, taking what kUnroll leaves over four at a time (and
-    the folding code beside it) was slower than one at a time."""
+    """Where a thread has more than a few vectors, taking what steps of 16 leave four at a time (and the
+    folding code beside it) was slower than one at a time, unless nearly a whole step is left."""
     got = child("""
 ctx, out = wg.Context(0), []
 for name, n in (("isamax", 24_000_000), ("isamax", 32_000_000), ("idamax", 20_000_000), ("idamax", 24_000_000),
-                ("isamax", 1), ("isamax", 1_000_000), ("idamax", 1_000_000)):
+                ("isamax", 1), ("isamax", 1_000_000), ("idamax", 1_000_000),
+                # a step of 16 vectors nearly whole, whole, and well short of it
+                ("idamax", 33_344_000), ("isamax", 4096 * 256 * 63), ("isamax", 4096 * 256 * 64),
+                ("idamax", 4096 * 256 * 32), ("isamax", 4096 * 256 * 60)):
     log, error = calls(lambda: getattr(ctx, name + "_dev")(n, P, 1, P))
     assert error is None, error
     out.append(next(line.split()[-1] for line in log if "reduce_vec" in line))
 print(json.dumps(out))
 """)
-    assert ["Lb1E" in name for name in got] == [True, False, True, False, True, True, True], got
+    assert ["Lb1E" in name for name in got] == [True, False, True, False] + [True] * 3 + [True, True] + [False] * 3, got
 
 
 def test_sgemm_k_groups_are_reached(child):

@@ -69,8 +69,17 @@ constexpr int kTail = 4;  // loads in flight over what is left of a range
 // kUnroll are too many (and may fold): us a call with / without, isamax 16 777 216
 // floats 14.5 / 15.8, 24 000 000 19.6 / 19.7, 32 328 320 25.9 / 24.1, 48 000 000
 // 33.4 / 31.9; dnrm2 6 000 000 doubles 13.0 / 13.8, 20 000 000 29.2 / 30.2,
-// 24 000 000 36.3 / 34.5.
+// 24 000 000 36.3 / 34.5. Also where what is left is a step of
+// kUnroll but for at most 1/32 of it (idamax 33 344 716 doubles 47.7 / 53.9).
 constexpr int kShortShare4 = 24, kShortShare8 = 20;
+
+template <typename T>
+bool short_share(int64_t n, int blocks) {
+  const int64_t threads = (int64_t)blocks * kThreads, step = kUnroll * (16 / (int64_t)sizeof(T));
+  return n <= threads * (sizeof(T) == 4 ? kShortShare4 : kShortShare8) ||
+         32 * (n % (threads * step)) >= 31 * threads * step;
+}
+
 constexpr int64_t kElemsPerBlockMin = 4096;
 // Up to this many first-pass blocks the last one to arrive folds (one launch).
 // The arrivals serialise on one word, about 10 ns each, and the fold comes
@@ -858,7 +867,7 @@ int launch_reduce(wgb_ctx *ctx, int64_t n, const typename Op::Elem *x, int64_t i
   int st;
   if ((st = fuse_fold(ctx, G, most, out.seq != 0, &fuse))) return st;
   const Output<Op> fused = fuse ? out : Output<Op>{nullptr, 0};
-  if (vec && n <= (int64_t)G * kThreads * (sizeof(typename Op::Elem) == 4 ? kShortShare4 : kShortShare8))
+  if (vec && short_share<typename Op::Elem>(n, G))
     reduce_vec<Op, true><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
   else if (vec)
     reduce_vec<Op, false><<<G, kThreads, 0, ctx->stream>>>(x, y, n, part, arrived, fused);
